@@ -1029,8 +1029,8 @@ def run_encoder(args, abi, ctx, decoder=False):
         meta = tdt_out["metadata"].download()
         decoded = {"avg_ms": decoder_ms, "tokens_per_window": [int(v) for v in meta[:active]],
                    **abi.decode_tdt_status(meta[stack.batch:stack.batch + active]),
-                   "kernel": "tdt_team_kernel" if tdt.team_size() > 1 else "tdt_decode_kernel",
-                   "workgroups_per_window": tdt.team_size(), "workgroups": active * tdt.team_size(),
+                   "kernel": "tdt_resident_kernel" if tdt.resident_windows() else
+                             "tdt_team_kernel" if tdt.team_size() > 1 else "tdt_decode_kernel",
                    "max_tokens": 1024}
     dense = None
     if not args.no_dense and not f32:

@@ -106,14 +106,24 @@ int pk_tdt_create(pk_context *ctx, const pk_tdt_desc *desc, pk_tdt_op **out);
 int pk_tdt_enqueue(pk_tdt_op *op, uint32_t active_batch, void *stream);
 int pk_tdt_enqueue_timed(pk_tdt_op *op, uint32_t active_batch, void *stream, void *start_event,
                          void *end_event);
-/* No reference counterpart: how many workgroups decode one window. 0
-   chooses (16 or 8 when every workgroup of the batch can be resident
-   together, else 1), 1 runs one workgroup per window, 8 and 16 split
-   every weight matrix over a team that meets at barriers in global memory
-   (bounded waits: a barrier that never completes sets the window's
-   PK_TDT_SYNC_TIMEOUT status). Results are bit-identical for every size.
-   Teams are built for the f16 profile: an f32 op always runs one
-   workgroup per window (0 chooses 1; 8 and 16 return PK_RANGE_ERROR).
+/* No reference counterpart: how many workgroups decode one window. 1 runs
+   one workgroup per window, 8 and 16 split every weight matrix over a team
+   that meets at barriers in global memory (bounded waits: a barrier that
+   never completes sets the window's PK_TDT_SYNC_TIMEOUT status), 0 leaves it
+   to the library: the resident decode (below) where it applies, and the size
+   that pk_tdt_team_size reports elsewhere (16 or 8 when every workgroup of
+   the batch can be resident together, else 1). Results are bit-identical in
+   every mode. Teams are built for the f16 profile: an f32 op reports 1, and
+   8 and 16 return PK_RANGE_ERROR.
+   The resident decode holds the decoder's weights in the LDS of one
+   workgroup on each of 160 (f16) or 214 (f32) compute units and decodes up to
+   16 (f16) or 6 (f32) windows per launch with them, up to four launches. Its
+   workgroups wait for each other, never without a bound: they give up after
+   10 ms at the start (another kernel holds their compute units) or after
+   2^20 polls later, and a kernel behind them in the stream then decodes the
+   windows with one workgroup each, so such a decode is late but complete and
+   never ends with PK_TDT_SYNC_TIMEOUT. Resident decodes of one process on one
+   GPU run one after the other (an event wait on the stream).
    A team launch is an ordinary launch whose grid fits the workgroups an
    idle device holds at once: kernels running on other streams at the same
    time can keep members from being resident, and a barrier that then
@@ -126,6 +136,11 @@ int pk_tdt_enqueue_timed(pk_tdt_op *op, uint32_t active_batch, void *stream, voi
    and leaves the team size as it was. */
 int pk_tdt_set_team_size(pk_tdt_op *op, uint32_t members);
 int pk_tdt_team_size(const pk_tdt_op *op, uint32_t *members);
+/* Windows of one resident launch of this op, 0 if it does not decode that
+   way; and the polls one of its waits makes before the launch is given up
+   (for tests: 0 gives up at the first unsuccessful poll). */
+int pk_tdt_resident_windows(const pk_tdt_op *op, uint32_t *windows);
+int pk_tdt_set_wait_limit(pk_tdt_op *op, uint32_t polls);
 /* Idempotent; frees the team buffers (after the device has drained), and
    enqueue after destroy returns PK_DESTROYED. Enqueue on a stream that is
    capturing a graph returns PK_INVALID_ARGUMENT. */

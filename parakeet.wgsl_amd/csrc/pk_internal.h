@@ -388,6 +388,10 @@ struct TdtArgs {
   uint32_t *tokens, *token_frames, *token_durations;  // [batch, max_tokens]
   uint32_t *counts, *status;     // [batch]
   uint32_t frames, max_tokens;
+  // tdt_decode_kernel behind resident launches: window b is decoded only if
+  // word 2 * (b / aborted_windows) * kTdtSyncStride is not 0 (null: always).
+  const uint32_t* aborted;
+  uint32_t aborted_windows;
 };
 // One workgroup per window; `f32` selects the f32 profile's kernel.
 hipError_t launch_tdt_decode(const TdtArgs& args, uint32_t batch, bool f32, hipStream_t stream,
@@ -411,6 +415,31 @@ bool tdt_team_members_supported(uint32_t members);
 uint32_t tdt_team_capacity(int device);
 hipError_t launch_tdt_team(const TdtArgs& args, const TdtTeam& team, uint32_t batch, hipStream_t stream,
                            hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
+
+// Resident decoding (pk_tdt_resident.hip, both profiles): the weights held in
+// the LDS of one workgroup per compute unit, all windows of a launch sharing
+// them; up to kTdtResidentLaunches launches of tdt_resident_windows() windows.
+// Each launch takes about as long as the longest of its windows; four of them
+// (64 f16 windows 24.8 ms, 24 f32 windows 20.9) still beat one workgroup per
+// window (36 and 49 ms), which takes any number of windows in one launch.
+constexpr uint32_t kTdtResidentLaunches = 4;
+constexpr uint32_t kTdtResidentBest = 216;  // words of one joint step: a member's best score or its turn
+// Exchange words of a window (64 bits each), two steps of each: h0 and h1 as
+// the gate chains read them, h1 in f32, the projection, the joint's words.
+constexpr uint32_t kTdtResidentH0 = 0, kTdtResidentH1F32 = 2 * kTdtHidden, kTdtResidentProjection = 4 * kTdtHidden,
+                   kTdtResidentHead = 6 * kTdtHidden,
+                   kTdtResidentWords = kTdtResidentHead + 2 * kTdtResidentBest;
+struct TdtResident {
+  uint32_t* sync;        // per launch: arrival count, abort flag, each kTdtSyncStride words apart
+  uint64_t* exchange;    // [batch, kTdtResidentWords], right after the sync words; cleared per decode
+  uint32_t base, windows;  // of one launch
+  uint32_t spin_limit;   // polls before a wait gives up
+  uint64_t join_ticks;   // 100 MHz ticks before the members stop waiting for each other at the start
+};
+uint32_t tdt_resident_windows(bool f32);
+bool tdt_resident_fits(int device, bool f32);
+hipError_t launch_tdt_resident(const TdtArgs& args, const TdtResident& resident, uint32_t batch, bool f32,
+                               hipStream_t stream, hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
 
 int conv_variant_count(bool f16);
 ConvGeometry conv_geometry(bool f16, int variant, uint32_t frames, uint32_t channels, uint32_t batch,

@@ -17,15 +17,17 @@ struct pk_tdt_op {
   std::string label;
   uint32_t batch = 0;
   pk::TdtArgs args{};
-  bool f32 = false;     // the f32 profile (one workgroup per window)
+  bool f32 = false;     // the f32 profile (no teams)
   pk::TdtTeam team{};   // members == 0: one workgroup per window
   uint32_t* team_memory = nullptr;
+  pk::TdtResident resident{};  // sync null: the team's or the window's own workgroups decode
   bool destroyed = false;
 };
 
 namespace {
 
 constexpr uint64_t H = PK_TDT_HIDDEN;
+constexpr int kMaxDevices = 64;
 
 // requireTensor (tdt-decoder.ts:458-478): the decoder tensor's size.
 int tensor(const void* p, uint64_t bytes, uint64_t need, const char* layout, const char* shape) {
@@ -103,13 +105,37 @@ uint32_t choose_members(int device, uint32_t batch, bool f32) {
 // Frees the team buffers once no launch can still use them (hipFree alone
 // would not order the free after work enqueued on another stream).
 void free_team(pk_tdt_op* op) {
-  if (op->team_memory) {
+  if (op->team_memory || op->resident.sync) {
     (void)hipSetDevice(op->ctx->device);
     (void)hipDeviceSynchronize();
     (void)hipFree(op->team_memory);
+    (void)hipFree(op->resident.sync);
   }
   op->team_memory = nullptr;
   op->team = pk::TdtTeam{};
+  op->resident = pk::TdtResident{};
+}
+
+// Gives an op whose team size was left to the library (0) the resident
+// decode, where the device holds its workgroups and the batch takes at most
+// kTdtResidentLaunches launches. Without memory for its exchange words (34
+// KB per window) the op decodes with the chosen team, as it does elsewhere.
+int set_resident(pk_tdt_op* op) {
+  const uint64_t windows = (uint64_t)pk::kTdtResidentLaunches * pk::tdt_resident_windows(op->f32);
+  if (op->batch > windows || op->ctx->device < 0 || op->ctx->device >= kMaxDevices || !pk::tdt_resident_fits(op->ctx->device, op->f32)) return PK_OK;
+  const uint64_t sync_words = 2ull * pk::kTdtResidentLaunches * pk::kTdtSyncStride;
+  uint32_t* memory = nullptr;
+  PK_HIP(hipSetDevice(op->ctx->device), "hipSetDevice");
+  if (hipMalloc(reinterpret_cast<void**>(&memory), sync_words * 4 + (uint64_t)op->batch * pk::kTdtResidentWords * 8) !=
+      hipSuccess) {
+    (void)hipGetLastError();
+    return PK_OK;
+  }
+  op->resident.sync = memory;
+  op->resident.exchange = reinterpret_cast<uint64_t*>(memory + sync_words);
+  op->resident.spin_limit = 1u << 20;    // each a memory round trip: about a second
+  op->resident.join_ticks = 1000000;     // 10 ms
+  return PK_OK;
 }
 
 int set_team(pk_tdt_op* op, uint32_t members) {
@@ -128,6 +154,28 @@ int set_team(pk_tdt_op* op, uint32_t members) {
   op->team.capacity = op->batch;
   op->team.spin_limit = 1u << 24;
   return PK_OK;
+}
+
+// Resident decodes of one GPU run one after the other: each wants a
+// workgroup on most compute units before it starts, and two that hold half
+// each would only time out. The event marks the end of the last one enqueued.
+struct ResidentTurn {
+  std::mutex mutex;
+  hipEvent_t last = nullptr;  // created at the first decode, kept until the process ends
+};
+ResidentTurn g_turns[kMaxDevices];
+
+hipError_t launch_in_turn(const pk_tdt_op* op, uint32_t batch, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
+  ResidentTurn& turn = g_turns[op->ctx->device];
+  std::lock_guard<std::mutex> lock(turn.mutex);
+  hipError_t e = hipSuccess;
+  if (turn.last)
+    e = hipStreamWaitEvent(stream, turn.last, 0);
+  else
+    e = hipEventCreateWithFlags(&turn.last, hipEventDisableTiming);
+  if (e == hipSuccess) e = pk::launch_tdt_resident(op->args, op->resident, batch, op->f32, stream, start, stop);
+  if (e == hipSuccess) e = hipEventRecord(turn.last, stream);
+  return e;
 }
 
 // Kernel arguments of a validated descriptor.
@@ -178,7 +226,6 @@ namespace {
 
 // The device address of `scratch` on each GPU, looked up once per device
 // with that device current (the host symbol is not a device address).
-constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mutex;
 uint32_t* g_scratch[kMaxDevices] = {};
 
@@ -221,7 +268,10 @@ int pk_tdt_create(pk_context* ctx, const pk_tdt_desc* d, pk_tdt_op** out) {
   op->batch = d->batch_size;
   op->args = args_of(d);
   op->f32 = d->precision == PK_PRECISION_F32;
-  if (int st = set_team(op, choose_members(ctx->device, op->batch, op->f32))) {
+  int st = set_team(op, choose_members(ctx->device, op->batch, op->f32));
+  if (st == PK_OK) st = set_resident(op);
+  if (st != PK_OK) {
+    free_team(op);
     delete op;
     return st;
   }
@@ -232,7 +282,8 @@ int pk_tdt_create(pk_context* ctx, const pk_tdt_desc* d, pk_tdt_op** out) {
 int pk_tdt_set_team_size(pk_tdt_op* op, uint32_t members) {
   if (!op) return fail(PK_INVALID_ARGUMENT, "TDT decoder op is null");
   if (op->destroyed) return fail(PK_DESTROYED, "%s was destroyed", op->label.c_str());
-  if (members == 0) members = choose_members(op->ctx->device, op->batch, op->f32);
+  const bool chosen = members == 0;
+  if (chosen) members = choose_members(op->ctx->device, op->batch, op->f32);
   else if (members == 1) members = 0;
   else if (!pk::tdt_team_members_supported(members))
     return fail(PK_RANGE_ERROR, "%s team size must be 0, 1, 8 or 16", op->label.c_str());
@@ -243,12 +294,26 @@ int pk_tdt_set_team_size(pk_tdt_op* op, uint32_t members) {
     return fail(PK_RANGE_ERROR, "%s: %u windows x %u workgroups cannot be resident together", op->label.c_str(),
                 op->batch, members);
   PK_HIP(hipSetDevice(op->ctx->device), "hipSetDevice");
-  return set_team(op, members);
+  if (int s = set_team(op, members)) return s;
+  return chosen ? set_resident(op) : PK_OK;
 }
 
 int pk_tdt_team_size(const pk_tdt_op* op, uint32_t* members) {
   if (!op || !members) return fail(PK_INVALID_ARGUMENT, "TDT decoder op or output is null");
   *members = op->team.members ? op->team.members : 1u;
+  return ok();
+}
+
+int pk_tdt_resident_windows(const pk_tdt_op* op, uint32_t* windows) {
+  if (!op || !windows) return fail(PK_INVALID_ARGUMENT, "TDT decoder op or output is null");
+  *windows = op->resident.sync ? pk::tdt_resident_windows(op->f32) : 0u;
+  return ok();
+}
+
+int pk_tdt_set_wait_limit(pk_tdt_op* op, uint32_t polls) {
+  if (!op) return fail(PK_INVALID_ARGUMENT, "TDT decoder op is null");
+  if (op->destroyed) return fail(PK_DESTROYED, "%s was destroyed", op->label.c_str());
+  op->resident.spin_limit = polls;
   return ok();
 }
 
@@ -271,6 +336,11 @@ int pk_tdt_enqueue_timed(pk_tdt_op* op, uint32_t active_batch, void* stream, voi
   PK_HIP(hipStreamIsCapturing(s, &capture), "hipStreamIsCapturing");
   if (capture != hipStreamCaptureStatusNone)
     return fail(PK_INVALID_ARGUMENT, "%s cannot be enqueued on a capturing stream", op->label.c_str());
+  if (op->resident.sync) {
+    PK_HIP(launch_in_turn(op, batch, s, static_cast<hipEvent_t>(start_event), static_cast<hipEvent_t>(end_event)),
+           "resident TDT decoder launch");
+    return ok();
+  }
   if (op->team.members) {
     // A refused team launch is an error: the op keeps its team size, and a
     // caller that wants one workgroup per window sets team size 1.

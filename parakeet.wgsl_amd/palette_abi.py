@@ -548,6 +548,8 @@ SIGNATURES = {
     "pk_tdt_destroy": (ctypes.c_int, [_VP]),
     "pk_tdt_release": (ctypes.c_int, [_VP]),
     "pk_tdt_set_team_size": (ctypes.c_int, [_VP, ctypes.c_uint32]),
+    "pk_tdt_resident_windows": (ctypes.c_int, [_VP, ctypes.POINTER(ctypes.c_uint32)]),
+    "pk_tdt_set_wait_limit": (ctypes.c_int, [_VP, ctypes.c_uint32]),
     "pk_graph_begin_capture": (ctypes.c_int, [_VP, _VP]),
     "pk_graph_end_capture": (ctypes.c_int, [_VP, _VP, _PPV]),
     "pk_graph_launch": (ctypes.c_int, [_VP, _VP]),
@@ -1254,13 +1256,24 @@ class TdtDecoderOp:
                                               start.handle if start else None, end.handle if end else None))
 
     def set_team_size(self, members: int) -> None:
-        """0 chooses, 1 runs one workgroup per window, 8 / 16 split each window over a team."""
+        """0 leaves it to the library (the resident decode where it applies), 1
+        runs one workgroup per window, 8 / 16 split each window over a team."""
         check(load().pk_tdt_set_team_size(self.handle, members))
 
     def team_size(self) -> int:
         out = ctypes.c_uint32()
         check(load().pk_tdt_team_size(self.handle, ctypes.byref(out)))
         return out.value
+
+    def resident_windows(self) -> int:
+        """Windows of one resident launch, 0 if the op does not decode that way."""
+        out = ctypes.c_uint32()
+        check(load().pk_tdt_resident_windows(self.handle, ctypes.byref(out)))
+        return out.value
+
+    def set_wait_limit(self, polls: int) -> None:
+        """Polls before a resident launch is given up (and decoded by one workgroup per window)."""
+        check(load().pk_tdt_set_wait_limit(self.handle, polls))
 
     def destroy(self) -> None:
         check(load().pk_tdt_destroy(self.handle))
