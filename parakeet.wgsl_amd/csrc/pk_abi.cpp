@@ -308,7 +308,6 @@ int find_variant(int precision, int family, int waves_m, int waves_n, int m_bloc
 // 96 x 128 on 3000-row 1024-wide GEMMs, 64 x 64 on 752 x 1024 and the
 // small-M kernel on the 375-row rel-pos linear; 96 x 128 also takes shapes
 // whose larger tiles would leave a costly partial round (3000-row QKV).
-// f32 keeps its own smallest-cost shape.
 Plan plan_launch(int precision, uint32_t rows, uint32_t inner, uint32_t columns, int cus) {
   if (precision == PK_PRECISION_F16) {
     auto pair_variant = [](int wn, int r, int c, int ks) {
@@ -397,18 +396,34 @@ Plan plan_launch(int precision, uint32_t rows, uint32_t inner, uint32_t columns,
     }
     return {best < 0 ? pair_variant(2, 6, 2, 2) : best, 1u};
   }
-  // f32: the largest tile that still fills the compute units.
+  // f32: the tile with the least predicted time, 4.5 us of launch plus per
+  // 1024 of K the time of a first workgroup on a compute unit and of each
+  // further one, as fitted to a sweep of every tile over 16 to 3008 rows of
+  // the encoder's GEMMs (within 15%). What it has to tell apart (us): 3008 x
+  // 1024 -> 4096 122 on 64 x 256 against 131 on 128 x 128 and 136 on 96 x 128;
+  // 3008 x 1024 -> 1024 39.1 on 96 x 128 against 42.5 and 43.4 on 32 and
+  // 64 x 128; 1504 x 1024 -> 1024 25.7 on 64 x 128 against 28.7 and 33.3;
+  // 188 x 1024 -> 4096 21.3 on 32 x 128 against 23.1 with K over four waves,
+  // which takes 188 x 4096 -> 1024 in 29.6 against 69.2.
+  struct Tile {
+    int wn, mb, nb, ks;
+    double first, each;
+  };
+  constexpr Tile kTiles[] = {{4, 1, 1, 1, 16.0, 14.0}, {4, 2, 1, 1, 20.5, 22.0}, {4, 3, 1, 1, 29.0, 32.0},
+                             {4, 4, 1, 1, 36.0, 43.0}, {4, 2, 2, 1, 34.5, 39.5}, {1, 1, 1, 4, 5.9, 5.9}};
   const int count = pk::f32_variant_count();
   int best = 0;
   double best_cost = 1e300;
   for (int i = 0; i < count; ++i) {
     const pk::TileShape s = shape_of(precision, i);
-    const double tiles = (double)pk::tiles_m(s, rows) * pk::tiles_n(s, columns);
-    const double rounds = std::ceil(tiles / cus);
-    const double cost = rounds * s.tile_rows() * s.tile_columns() * (1.0 + 0.25 / s.m_blocks);
-    if (cost < best_cost * 0.999) {
-      best_cost = cost;
-      best = i;
+    for (const Tile& t : kTiles) {
+      if (t.wn != s.waves_n || t.mb != s.m_blocks || t.nb != s.n_blocks || t.ks != s.k_split) continue;
+      const double tiles = (double)pk::tiles_m(s, rows) * pk::tiles_n(s, columns);
+      const double cost = 4.5 + (t.first + (std::ceil(tiles / cus) - 1.0) * t.each) * inner / 1024.0;
+      if (cost < best_cost * 0.999) {
+        best_cost = cost;
+        best = i;
+      }
     }
   }
   return {best, 1u};

@@ -1,18 +1,42 @@
-// pk_gemm_f32.hip - fused palette-weight GEMM, f32 operands and f32 MFMA
-// (v_mfma_f32_32x32x2_f32) for gfx950: the FP32 twin of pk_gemm_f16.hip
-// (reference: src/webgpu/kernels/gemm.ts:2356-2599, epilogue :2847-2869).
+// pk_gemm_f32.hip - fused palette-weight GEMM with f32 operands for gfx950:
+// the FP32 twin of pk_gemm_f16.hip (reference:
+// src/webgpu/kernels/gemm.ts:2356-2599, epilogue :2847-2869).
 //
-// Same operand-order codes as the f16 kernel: in MFMA step s (0..31) of a
-// 64-deep K block, lane half h stands for k = 64*kb + 32*h + s in both
-// operands, which is code u = s of the lane's 32-code stream. One decoded
-// code per lane feeds one MFMA per row block, so decode work is small next
-// to the 64-cycle f32 MFMA.
+// The f32 matrix units are 16 times slower than the bf16 ones, so every f32
+// operand is split into three bf16 terms that add up to it exactly, and six
+// of the nine products of terms go through v_mfma_f32_32x32x16_bf16 into one
+// f32 accumulator, smallest first; the three left out are below 2^-24 of the
+// product. One accumulator addition per 16 k instead of one per 2 k leaves the
+// sums nearer to 64 bits than the f32 units' (norm-wise 4.9e-7 against 5.7e-7
+// at K = 1024, 1.0e-6 against 1.1e-6 at K = 4096, 2.4e-7 and 5.0e-7 with K over
+// four waves).
+//
+// Bound: the bf16 matrix units in principle (a sixth of their rate: 417
+// TFLOP/s nominal, about 190 at the rate of a large library product), LDS
+// reads and the per-step chain in practice. A wave's operands for the next
+// 16 k are gathered and read during the products of the current ones, the A
+// tile is split once per workgroup on its way into a ring of three LDS
+// buffers (32 k each, one barrier per step), and all loads are unconditional
+// (a branch around one ends the compiler's scheduling region: 24.3 -> 20.6 us
+// at 188 x 1024 -> 4096). The palette lies in LDS as split entries: one 8-byte
+// gather per code and three byte permutes per pair.
+//
+// Against v_mfma_f32_32x32x2_f32 before: 3008 x 1024 -> 4096 (5-bit) 214 ->
+// 122 us (206 TFLOP/s), 3008 x 4096 -> 1024 227 -> 135, 3008 x 1024 -> 3072 168
+// -> 99, 256 x 1024 -> 4096 (6-bit) 30.5 -> 22.5, 188 x 4096 -> 1024 102 -> 30,
+// 16 x 1024 -> 4096 28 -> 10.
+//
+// Codes in operand order: lane half h owns k = 64 kb + 32 h + u, so MFMA
+// sub-step s (0..3) multiplies codes u = 8 s + [0, 8) of both halves.
 #include "pk_internal.h"
 
 namespace pk {
 namespace {
 
 typedef float float16v __attribute__((ext_vector_type(16)));
+typedef float float2v __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 template <int BITS>
 __device__ __forceinline__ uint32_t lane_code(const uint32_t* w, int u) {
@@ -33,25 +57,51 @@ __device__ __forceinline__ float silu(float v) {
   return v * __builtin_amdgcn_rcpf(1.0f + e);
 }
 
-template <int BITS, int WM, int WN, int MB, int NB>
-__global__ __launch_bounds__(64 * WM * WN) void gemm_f32_kernel(GemmArgs args) {
-  constexpr int T = 64 * WM * WN;
-  constexpr int BM = 32 * WM * MB;
+// Two f32 values rounded to bf16, the first in the low half.
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
+  const bf16x2 p = __builtin_convertvector((float2v{a, b}), bf16x2);
+  return __builtin_bit_cast(uint32_t, p);
+}
+__device__ __forceinline__ float low_f32(uint32_t p) { return __uint_as_float(p << 16); }
+__device__ __forceinline__ float high_f32(uint32_t p) { return __uint_as_float(p & 0xffff0000u); }
+
+// Two f32 values as three bf16 terms each, rounded to nearest one after the
+// other: the sum of the three is the value (8 + 8 + 8 significand bits).
+struct Split {
+  uint32_t hi, mid, lo;
+};
+__device__ __forceinline__ Split split2(float a, float b) {
+  Split s;
+  s.hi = pack_bf16(a, b);
+  const float ra = a - low_f32(s.hi), rb = b - high_f32(s.hi);
+  s.mid = pack_bf16(ra, rb);
+  s.lo = pack_bf16(ra - low_f32(s.mid), rb - high_f32(s.mid));
+  return s;
+}
+
+template <int BITS, int WN, int MB, int NB, int KS>
+__global__ __launch_bounds__(64 * WN * KS, 2) void gemm_f32_kernel(GemmArgs args) {
+  static_assert(KS == 1 || (WN == 1 && MB == 1 && NB == 1 && KS == 4), "K over the four waves of one 32 x 32 tile");
+  constexpr int T = 64 * WN * KS;  // threads, GT of them share a K block
+  constexpr int GT = T / KS;
+  constexpr int BM = 32 * MB;
   constexpr int BN = 32 * WN * NB;
   constexpr int E = 1 << BITS;
   constexpr int LUT_CAP = (BN / 16 + 2) * E;
-  constexpr int ROW_BYTES = 256;  // 64 floats of one row per K step
-  constexpr int CH = BM * 16 / T;
-  static_assert(BM * 16 % T == 0, "A tile chunks must divide evenly");
+  constexpr int PLANE = BM * 64;  // bytes of one term of a step's A tile: 32 k per row
+  constexpr int CH = BM * 8 / GT;  // runs of 4 k per thread
+  static_assert(BM * 8 % GT == 0, "the A tile divides evenly");
 
-  __shared__ __attribute__((aligned(16))) uint8_t a_lds[2][BM * ROW_BYTES];
-  __shared__ float lut_lds[LUT_CAP];
+  __shared__ __align__(16) uint8_t a_lds_all[KS][3][3 * PLANE];
+  __shared__ uint2 lut_lds[LUT_CAP];  // {hi | mid << 16, lo}
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
-  const int wave_m = wave / WN;
-  const int wave_n = wave % WN;
+  const int wave_n = KS > 1 ? 0 : wave;
+  const uint32_t part = KS > 1 ? wave : 0;  // this wave's K blocks: part, part + KS, ...
+  const int gtid = KS > 1 ? lane : tid;
+  auto& a_lds = a_lds_all[part];
   const int j = lane & 31;
   const int h = lane >> 5;
 
@@ -67,69 +117,67 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_kernel(GemmArgs args) {
   const uint32_t G = args.palette_groups;
   const uint32_t g_lo = min(n0 / gc, G - 1u);
   const uint32_t g_hi = min((min(n0 + BN, N) - 1u) / gc, G - 1u);
-  {
-    const uint32_t entries = (g_hi - g_lo + 1u) * E;
-    const float* src = static_cast<const float*>(args.palette) + (uint64_t)g_lo * E;
-    for (uint32_t i = tid; i < entries; i += T) lut_lds[i] = src[i];
-  }
-  const float* lut_col[NB];
-#pragma unroll
-  for (int ni = 0; ni < NB; ++ni) {
-    const uint32_t n = n0 + (wave_n * NB + ni) * 32 + j;
-    const uint32_t g = min(n / gc, G - 1u) - g_lo;
-    lut_col[ni] = lut_lds + g * E;
-  }
+  const float* palette = static_cast<const float*>(args.palette);
 
   const uint32_t nb0 = n0 / 32u + wave_n * NB;
   uint32_t cw[NB][BITS];
   auto load_codes = [&](uint32_t kb, uint32_t (&dst)[NB][BITS]) {
 #pragma unroll
     for (int ni = 0; ni < NB; ++ni) {
-      const uint32_t nb = nb0 + ni;
-      if (nb < n_blocks_total) {
-        const uint32_t* blk = args.codes + ((uint64_t)nb * k_blocks + kb) * block_words(BITS);
-        const uint4 p0 = reinterpret_cast<const uint4*>(blk)[lane];
-        dst[ni][0] = p0.x;
-        dst[ni][1] = p0.y;
-        dst[ni][2] = p0.z;
-        dst[ni][3] = p0.w;
-        if constexpr (BITS == 5) {
-          dst[ni][4] = blk[256 + lane];
-        } else {
-          const uint2 p1 = reinterpret_cast<const uint2*>(blk + 256)[lane];
-          dst[ni][4] = p1.x;
-          dst[ni][5] = p1.y;
-        }
+      const uint32_t nb = min(nb0 + ni, n_blocks_total - 1u);  // past the end: columns never stored
+      const uint32_t* blk = args.codes + ((uint64_t)nb * k_blocks + kb) * block_words(BITS);
+      const uint4 p0 = reinterpret_cast<const uint4*>(blk)[lane];
+      dst[ni][0] = p0.x;
+      dst[ni][1] = p0.y;
+      dst[ni][2] = p0.z;
+      dst[ni][3] = p0.w;
+      if constexpr (BITS == 5) {
+        dst[ni][4] = blk[256 + lane];
       } else {
-#pragma unroll
-        for (int q = 0; q < BITS; ++q) dst[ni][q] = 0u;
+        const uint2 p1 = reinterpret_cast<const uint2*>(blk + 256)[lane];
+        dst[ni][4] = p1.x;
+        dst[ni][5] = p1.y;
       }
     }
   };
 
+  // Step t = 2 kb + half: the k of MFMA sub-steps 2 half and 2 half + 1, i.e.
+  // 64 kb + 32 h + 16 half + [0, 16) for both lane halves h, as eight runs of
+  // four per row. Loads are unconditional: a row past the end repeats the
+  // last one (never stored), a run past K is zeroed.
   const float* a_ptr = static_cast<const float*>(args.a);
-  uint4 a_stage[CH];
-  auto load_a = [&](uint32_t kb) {
+  const uint32_t own_blocks = k_blocks > part ? (k_blocks - part + KS - 1u) / KS : 0u;
+  const uint32_t steps = 2u * own_blocks;
+  float4 a_stage[2][CH];
+  auto run_k = [&](uint32_t t, int run) {
+    return ((t >> 1) * KS + part) * 64u + (t & 1u) * 16u + ((run >> 2) * 32 + (run & 3) * 4);
+  };
+  auto load_a = [&](uint32_t t, float4 (&stage)[CH]) {
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-      const int idx = tid + c * T;
-      const int r = idx >> 4;
-      const int ch = idx & 15;
-      const uint32_t m = m0 + r;
-      const uint32_t k = kb * 64u + ch * 4u;
-      if (m < M && k < K)
-        a_stage[c] = *reinterpret_cast<const uint4*>(a_ptr + (uint64_t)m * K + k);
-      else
-        a_stage[c] = make_uint4(0u, 0u, 0u, 0u);
+      const int idx = gtid + c * GT;
+      const uint32_t m = min(m0 + (idx >> 3), M - 1u);
+      const uint32_t k = min(run_k(t, idx & 7), K - 4u);
+      stage[c] = *reinterpret_cast<const float4*>(a_ptr + (uint64_t)m * K + k);
     }
   };
-  auto store_a = [&](int buf) {
+  // A row of a term is 64 bytes, chunk 2 s + h of 16 for sub-step s and lane
+  // half h; rows four apart start at the same bank, so the chunk is XORed
+  // with bits 2 and 3 of the row.
+  auto store_a = [&](uint32_t t, uint32_t buf, const float4 (&stage)[CH]) {
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-      const int idx = tid + c * T;
-      const int r = idx >> 4;
-      const int ch = idx & 15;
-      *reinterpret_cast<uint4*>(&a_lds[buf][r * ROW_BYTES + ((ch ^ (r & 7)) << 4)]) = a_stage[c];
+      const int idx = gtid + c * GT;
+      const int r = idx >> 3, run = idx & 7;
+      const bool inside = run_k(t, run) < K;
+      const float4 x = stage[c];
+      const Split s0 = split2(inside ? x.x : 0.0f, inside ? x.y : 0.0f);
+      const Split s1 = split2(inside ? x.z : 0.0f, inside ? x.w : 0.0f);
+      const int chunk = ((run >> 1) & 1) * 2 + (run >> 2);
+      uint8_t* dst = &a_lds[buf][r * 64 + ((chunk ^ ((r >> 2) & 3)) << 4) + (run & 1) * 8];
+      *reinterpret_cast<uint2*>(dst) = make_uint2(s0.hi, s1.hi);
+      *reinterpret_cast<uint2*>(dst + PLANE) = make_uint2(s0.mid, s1.mid);
+      *reinterpret_cast<uint2*>(dst + 2 * PLANE) = make_uint2(s0.lo, s1.lo);
     }
   };
 
@@ -141,65 +189,208 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_kernel(GemmArgs args) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[mi][ni][v] = 0.0f;
 
-  load_codes(0, cw);
-  load_a(0);
-  store_a(0);
-  __syncthreads();
+  if (steps) {
+    load_a(0, a_stage[0]);
+    load_codes(part, cw);
+    load_a(1, a_stage[1]);
+  }
+  {
+    const uint32_t entries = (g_hi - g_lo + 1u) * E;
+    for (uint32_t i = tid; i < entries; i += T) {
+      const Split s = split2(palette[(uint64_t)g_lo * E + i], 0.0f);
+      lut_lds[i] = make_uint2((s.hi & 0xffffu) | s.mid << 16, s.lo & 0xffffu);
+    }
+  }
+  uint32_t lut_base[NB];  // first entry of the lane's column's palette group
+#pragma unroll
+  for (int ni = 0; ni < NB; ++ni) {
+    const uint32_t n = n0 + (wave_n * NB + ni) * 32 + j;
+    lut_base[ni] = (min(min(n / gc, G - 1u), g_hi) - g_lo) * E;
+  }
+  // Weights of a sub-step: the entries of its eight codes per column block,
+  // then the three operands.
+  auto gather = [&](const uint32_t (&c)[NB][BITS], int sub, uint2 (&e)[NB][8]) {
+#pragma unroll
+    for (int ni = 0; ni < NB; ++ni)
+#pragma unroll
+      for (int u = 0; u < 8; ++u) e[ni][u] = lut_lds[lut_base[ni] + lane_code<BITS>(c[ni], sub * 8 + u)];
+  };
+  auto assemble = [&](const uint2 (&e)[NB][8], bf16x8 (&w)[NB][3]) {
+#pragma unroll
+    for (int ni = 0; ni < NB; ++ni) {
+      uint32_t hi[4], mid[4], lo[4];
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const uint2 e0 = e[ni][2 * p], e1 = e[ni][2 * p + 1];
+        hi[p] = __builtin_amdgcn_perm(e1.x, e0.x, 0x05040100u);
+        mid[p] = __builtin_amdgcn_perm(e1.x, e0.x, 0x07060302u);
+        lo[p] = __builtin_amdgcn_perm(e1.y, e0.y, 0x05040100u);
+      }
+      w[ni][0] = __builtin_bit_cast(bf16x8, make_uint4(hi[0], hi[1], hi[2], hi[3]));
+      w[ni][1] = __builtin_bit_cast(bf16x8, make_uint4(mid[0], mid[1], mid[2], mid[3]));
+      w[ni][2] = __builtin_bit_cast(bf16x8, make_uint4(lo[0], lo[1], lo[2], lo[3]));
+    }
+  };
+  auto read_a = [&](uint32_t buf, int s, bf16x8 (&a)[MB][3]) {
+#pragma unroll
+    for (int mi = 0; mi < MB; ++mi) {
+      const int r = mi * 32 + j;
+      const uint8_t* src = &a_lds[buf][r * 64 + (((2 * s + h) ^ ((r >> 2) & 3)) << 4)];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) a[mi][q] = *reinterpret_cast<const bf16x8*>(src + q * PLANE);
+    }
+  };
+  // the smallest products first
+  auto multiply = [&](const bf16x8 (&w)[NB][3], const bf16x8 (&a)[MB][3]) {
+    constexpr int kTerms[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
+#pragma unroll
+    for (int t = 0; t < 6; ++t)
+#pragma unroll
+      for (int mi = 0; mi < MB; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < NB; ++ni)
+          acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[ni][kTerms[t][0]], a[mi][kTerms[t][1]], acc[mi][ni],
+                                                               0, 0, 0);
+  };
 
-  for (uint32_t kb = 0; kb < k_blocks; ++kb) {
-    const int buf = kb & 1;
-    const bool more = kb + 1 < k_blocks;
-    uint32_t cn[NB][BITS];
-    if (more) {
-      load_codes(kb + 1, cn);
-      load_a(kb + 1);
+  // A wave that has a K block to itself needs no barrier: its LDS operations
+  // complete in order.
+  auto sync = [&] {
+    if constexpr (KS == 1) {
+      __syncthreads();
+    } else {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
     }
-    const uint8_t* tile = a_lds[buf];
+  };
+  if constexpr (KS > 1) __syncthreads();  // the palette
+  if (steps) {
+    store_a(0, 0, a_stage[0]);
+    load_a(min(2u, steps - 1u), a_stage[0]);
+    store_a(1, 1, a_stage[1]);
+    load_a(min(3u, steps - 1u), a_stage[1]);
+    sync();
+
+    // Step t multiplies buffer t % 3 while t + 1 is read for its first
+    // sub-step and t + 2 is written; each sub-step's operands are fetched
+    // during the products of the one before.
+    bf16x8 w[NB][3], a0[MB][3], a1[MB][3];
+    uint2 e[NB][8];
+    uint32_t buf = 0;
+    gather(cw, 0, e);
+    read_a(0, 0, a0);
+    assemble(e, w);
+    for (uint32_t i = 0; i < own_blocks; ++i) {
+      uint32_t cn[NB][BITS];
+      load_codes(min(i + 1u, own_blocks - 1u) * KS + part, cn);
 #pragma unroll
-    for (int s4 = 0; s4 < 8; ++s4) {
-      float4 af[MB];
-#pragma unroll
-      for (int mi = 0; mi < MB; ++mi) {
-        const int r = (wave_m * MB + mi) * 32 + j;
-        const int ch = h * 8 + s4;
-        af[mi] = *reinterpret_cast<const float4*>(&tile[r * ROW_BYTES + ((ch ^ (r & 7)) << 4)]);
+      for (int half = 0; half < 2; ++half) {
+        const uint32_t t = 2u * i + half;
+        const uint32_t buf1 = buf == 2u ? 0u : buf + 1u, buf2 = buf1 == 2u ? 0u : buf1 + 1u;
+        gather(cw, 2 * half + 1, e);
+        read_a(buf, 1, a1);
+        multiply(w, a0);
+        assemble(e, w);
+        if (half == 0)
+          gather(cw, 2, e);
+        else
+          gather(cn, 0, e);
+        read_a(buf1, 0, a0);
+        store_a(min(t + 2u, steps - 1u), buf2, a_stage[half]);
+        load_a(min(t + 4u, steps - 1u), a_stage[half]);
+        multiply(w, a1);
+        assemble(e, w);
+        sync();
+        buf = buf1;
       }
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        float bw[NB];
-#pragma unroll
-        for (int ni = 0; ni < NB; ++ni) bw[ni] = lut_col[ni][lane_code<BITS>(cw[ni], s4 * 4 + t)];
-#pragma unroll
-        for (int mi = 0; mi < MB; ++mi) {
-          const float a = t == 0 ? af[mi].x : t == 1 ? af[mi].y : t == 2 ? af[mi].z : af[mi].w;
-#pragma unroll
-          for (int ni = 0; ni < NB; ++ni)
-            acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x2f32(bw[ni], a, acc[mi][ni], 0, 0, 0);
-        }
-      }
-    }
-    if (more) {
-      store_a(buf ^ 1);
 #pragma unroll
       for (int ni = 0; ni < NB; ++ni)
 #pragma unroll
         for (int q = 0; q < BITS; ++q) cw[ni][q] = cn[ni][q];
     }
+  }
+
+  // A value that is infinite, NaN or rounds up past the largest bf16 has no
+  // split: its rows or columns come out as NaN or infinity. A wave that
+  // finds one computes its blocks again on the f32 units, one code and one
+  // element of A per lane and MFMA.
+  bool finite = true;
+#pragma unroll
+  for (int mi = 0; mi < MB; ++mi)
+#pragma unroll
+    for (int ni = 0; ni < NB; ++ni)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) finite &= __builtin_fabsf(acc[mi][ni][v]) <= 3.402823466e+38f;
+  if (!__all(finite)) {
+#pragma unroll 1
+    for (int ni = 0; ni < NB; ++ni) {
+      const uint32_t n = n0 + (wave_n * NB + ni) * 32 + j;
+      const float* lut = palette + (uint64_t)min(n / gc, G - 1u) * E;
+      const uint32_t nb = min(nb0 + ni, n_blocks_total - 1u);
+#pragma unroll 1
+      for (int mi = 0; mi < MB; ++mi) {
+        const uint32_t m = m0 + mi * 32 + j;
+        float16v c;
+        for (int v = 0; v < 16; ++v) c[v] = 0.0f;
+        for (uint32_t kb = part; kb < k_blocks; kb += KS) {
+          const uint32_t* blk = args.codes + ((uint64_t)nb * k_blocks + kb) * block_words(BITS);
+          uint32_t words[BITS + 1];
+          for (int q = 0; q < 4; ++q) words[q] = blk[lane * 4 + q];
+          for (int q = 4; q < BITS; ++q) words[q] = blk[256 + lane * (BITS - 4) + q - 4];
+          words[BITS] = 0u;
+#pragma unroll
+          for (int s = 0; s < 32; ++s) {
+            const uint32_t k = kb * 64u + h * 32u + s;
+            const float x = m < M && k < K ? a_ptr[(uint64_t)m * K + k] : 0.0f;
+            c = __builtin_amdgcn_mfma_f32_32x32x2f32(lut[lane_code<BITS>(words, s)], x, c, 0, 0, 0);
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+          for (int o = 0; o < NB; ++o)
+            if (i == mi && o == ni) acc[i][o] = c;
+      }
+    }
+  }
+
+  if constexpr (KS > 1) {
+    // The parts meet in LDS; wave q sums quad q of every column block in part
+    // order.
     __syncthreads();
+    float4* partial = reinterpret_cast<float4*>(a_lds_all);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      partial[(wave * 4 + q) * 64 + lane] =
+          make_float4(acc[0][0][4 * q], acc[0][0][4 * q + 1], acc[0][0][4 * q + 2], acc[0][0][4 * q + 3]);
+    __syncthreads();
+    float4 sum = partial[wave * 64 + lane];
+#pragma unroll
+    for (int p = 1; p < KS; ++p) {
+      const float4 v = partial[(p * 4 + wave) * 64 + lane];
+      sum.x += v.x;
+      sum.y += v.y;
+      sum.z += v.z;
+      sum.w += v.w;
+    }
+    acc[0][0][0] = sum.x;
+    acc[0][0][1] = sum.y;
+    acc[0][0][2] = sum.z;
+    acc[0][0][3] = sum.w;
   }
 
   float* out = static_cast<float*>(args.out);
   const float* residual = static_cast<const float*>(args.residual);
 #pragma unroll
   for (int mi = 0; mi < MB; ++mi) {
-    const uint32_t m = m0 + (wave_m * MB + mi) * 32 + j;
+    const uint32_t m = m0 + mi * 32 + j;
     if (m >= M) continue;
 #pragma unroll
     for (int ni = 0; ni < NB; ++ni) {
       const uint32_t nbase = n0 + (wave_n * NB + ni) * 32 + h * 4;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const uint32_t n = nbase + q * 8;
+      for (int q = 0; q < (KS > 1 ? 1 : 4); ++q) {
+        const uint32_t n = nbase + (KS > 1 ? wave : q) * 8;
         if (n >= N) continue;
         float v[4];
 #pragma unroll
@@ -240,19 +431,20 @@ struct Variant {
   void (*kernel6)(GemmArgs);
 };
 
-#define PK_F32_VARIANT(WM, WN, MB, NB)                                             \
-  Variant {                                                                        \
-    TileShape{WM, WN, MB, NB}, "pk_gemm_f32_b5_w" #WM "x" #WN "_m" #MB "n" #NB,    \
-        "pk_gemm_f32_b6_w" #WM "x" #WN "_m" #MB "n" #NB,                           \
-        gemm_f32_kernel<5, WM, WN, MB, NB>, gemm_f32_kernel<6, WM, WN, MB, NB>     \
+#define PK_F32_VARIANT(WN, MB, NB, KS)                                                                 \
+  Variant {                                                                                            \
+    TileShape{1, WN, MB, NB, KS}, "pk_gemm_f32_b5_n" #WN "k" #KS "_m" #MB "n" #NB,                   \
+        "pk_gemm_f32_b6_n" #WN "k" #KS "_m" #MB "n" #NB, gemm_f32_kernel<5, WN, MB, NB, KS>, \
+        gemm_f32_kernel<6, WN, MB, NB, KS>                                                          \
   }
 
 const Variant kVariants[] = {
-    PK_F32_VARIANT(1, 4, 1, 1),  // 32 x 128
-    PK_F32_VARIANT(1, 4, 2, 1),  // 64 x 128
-    PK_F32_VARIANT(1, 4, 2, 2),  // 64 x 256
-    PK_F32_VARIANT(2, 2, 2, 2),  // 128 x 128
-    PK_F32_VARIANT(1, 2, 1, 1),  // 32 x 64
+    PK_F32_VARIANT(4, 1, 1, 1),  // 32 x 128
+    PK_F32_VARIANT(4, 2, 1, 1),  // 64 x 128
+    PK_F32_VARIANT(4, 3, 1, 1),  // 96 x 128
+    PK_F32_VARIANT(4, 4, 1, 1),  // 128 x 128
+    PK_F32_VARIANT(4, 2, 2, 1),  // 64 x 256
+    PK_F32_VARIANT(1, 1, 1, 4),  // 32 x 32, K over four waves
 };
 
 }  // namespace

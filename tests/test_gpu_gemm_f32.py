@@ -1,0 +1,83 @@
+"""The f32 palette GEMM's split product (three bf16 terms per operand) on
+every tile: edges of the tiles and K tails, several palette groups in one
+tile, and operands that have no split (infinite, NaN, beyond the largest
+bf16), which come from the f32 matrix units instead."""
+import numpy as np
+import pytest
+
+from test_gpu_parity import Scope, run_case
+
+pytestmark = pytest.mark.gpu
+
+# Norm-wise error of an f32 sum of K products: each addition rounds by at most
+# 2^-24 of a partial sum, sqrt(K) of them as a random walk; the split leaves
+# out 2^-24 of a product. 4 x sqrt(4096) x 2^-24 covers every K here.
+TOLERANCE = 1.6e-5
+
+
+@pytest.fixture
+def scope(ctx):
+    s = Scope(ctx)
+    yield s
+    s.close()
+
+
+def exact(workloads, case):
+    codes = case.weight.codes.astype(np.int64)
+    lut = case.weight.palette.astype(np.float64).reshape(-1, 1 << case.weight.bits)
+    n = codes.shape[1]
+    group = np.minimum(np.arange(n) // max(n // lut.shape[0], 1), lut.shape[0] - 1)
+    with np.errstate(invalid="ignore", over="ignore"):
+        y = case.a.astype(np.float64) @ lut[group[None, :], codes]
+        if case.bias is not None:
+            y = y + case.bias.astype(np.float64)
+        if case.activation == "relu":
+            y = np.maximum(y, 0)
+    return y
+
+
+@pytest.mark.parametrize("rows,inner,columns,bits,groups", [
+    (1, 64, 128, 5, 1), (31, 32, 16, 6, 1), (33, 96, 160, 5, 1), (65, 160, 272, 6, 1), (97, 192, 96, 6, 3),
+    (129, 320, 384, 5, 3), (193, 1024, 528, 6, 1), (40, 4096, 64, 5, 1)])
+def test_split_product_on_every_tile(abi, ctx, scope, workloads, rows, inner, columns, bits, groups):
+    case = workloads.gemm_case(rows + inner, rows, inner, columns, bits, dtype=np.float32, groups=groups,
+                               bias=True, activation="relu" if rows % 2 else "none")
+    want = exact(workloads, case)
+    for variant in [None] + list(range(abi.variant_count("f32"))):
+        got = run_case(abi, ctx, scope, case, variant=variant)
+        error = np.linalg.norm(got - want) / np.linalg.norm(want)
+        print(rows, inner, columns, "variant", variant, "error", error, flush=True)
+        assert error <= TOLERANCE
+
+
+def test_wide_range_of_magnitudes(abi, ctx, scope, workloads):
+    """Rows scaled from 1e-30 to 1e30: each row's own error stays that of f32."""
+    case = workloads.gemm_case(3, 61, 256, 128, 5, dtype=np.float32)
+    case.a *= (10.0 ** np.arange(-30, 31)[:, None]).astype(np.float32)
+    want = exact(workloads, case)
+    for variant in range(abi.variant_count("f32")):
+        got = run_case(abi, ctx, scope, case, variant=variant).astype(np.float64)
+        assert (np.linalg.norm(got - want, axis=1) <= TOLERANCE * np.linalg.norm(want, axis=1)).all()
+
+
+@pytest.mark.parametrize("where", ["a", "palette"])
+def test_operands_without_a_split(abi, ctx, scope, workloads, where):
+    """Infinity, NaN and 3.4e38 in A or in the palette: the outputs are what
+    f32 arithmetic gives (infinities of the right sign, NaN where they meet)
+    and the rows and columns without them keep their values."""
+    case = workloads.gemm_case(9, 70, 192, 160, 5, dtype=np.float32)
+    if where == "a":
+        case.a[3, 5], case.a[40, 100], case.a[65, 7], case.a[69, 191] = np.inf, np.nan, -np.inf, 3.4e38
+    else:
+        case.weight.palette[...] = np.where(np.arange(32) == 7, np.inf, case.weight.palette)
+        case.weight.codes[:, 3:] = np.where(case.weight.codes[:, 3:] == 7, 8, case.weight.codes[:, 3:])
+        case.weight.packed[...] = workloads.pack_codes(case.weight.codes, 5)
+    want = exact(workloads, case)
+    finite = np.isfinite(want)
+    assert 0 < finite.sum() < finite.size
+    for variant in range(abi.variant_count("f32")):
+        got = run_case(abi, ctx, scope, case, variant=variant)
+        np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+        np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)].astype(np.float32))
+        error = np.abs(got[finite] - want[finite]) / np.maximum(np.abs(want[finite]), 1.0)
+        assert error.max() <= TOLERANCE
