@@ -296,18 +296,19 @@ int find_variant(int precision, int family, int waves_m, int waves_n, int m_bloc
 // Launch planner. The f16 choice follows MI355X measurements of every
 // compiled tile shape over the encoder's GEMM shapes (M 1..3008, K
 // 1024/4096, N 1024..4096, the rel-pos linear's 2T-1 rows). Up to 64 rows,
-// and up to 256 rows of a deep-K (K >= 2048) or at most 1024 columns wide
-// GEMM, the small-M kernel (32-row blocks, K round robin over eight
-// wavefronts) wins (output projection at 188 rows: 5.96 us against 7.88 us
-// for the 64 x 64 pair-code tile); up to 256 rows otherwise the 64 x 64
-// pair-code tile (FF expand at 188 rows: 8.30 us against 8.84 us for the
-// best small-M shape); deep-K shapes take 96 x 64 while
+// and while its 32 x 32 tiles fit one round of the compute units (two rounds
+// of a deep-K GEMM, K >= 2048), the small-M kernel (32-row blocks, K round
+// robin over eight wavefronts) wins (188 x 1024 -> 1024: 5.7 us against 8.2
+// for the 64 x 64 pair-code tile; 300 x 1024 -> 640 5.4 against 7.9); up to 256
+// rows otherwise the 64 x 64 pair-code tile (188 x 1024 -> 2048 8.0 us against
+// 8.9, -> 4096 8.2 against 12.7); deep-K shapes take 64 x 64 and 96 x 64 while
 // those fill the chip and 96 x 128 beyond. Every other shape takes the
 // candidate with the least (rounds of workgroups) x (measured time of one
 // workgroup), which puts 192 x 128 on the FF expand and convolution PW1,
-// 96 x 128 on 3000-row 1024-wide GEMMs, 64 x 64 on 752 x 1024 and the
-// small-M kernel on the 375-row rel-pos linear; 96 x 128 also takes shapes
-// whose larger tiles would leave a costly partial round (3000-row QKV).
+// 96 x 128 on 3000-row 1024-wide GEMMs and 64 x 64 on 752 x 1024 and the
+// 375-row rel-pos linear (8.4 us against 8.9 for a 64 x 32 small-M tile);
+// 96 x 128 also takes shapes whose larger tiles would leave a costly partial
+// round (3000-row QKV).
 Plan plan_launch(int precision, uint32_t rows, uint32_t inner, uint32_t columns, int cus) {
   if (precision == PK_PRECISION_F16) {
     auto pair_variant = [](int wn, int r, int c, int ks) {
@@ -318,18 +319,18 @@ Plan plan_launch(int precision, uint32_t rows, uint32_t inner, uint32_t columns,
       return (uint64_t)((rows + tile_rows - 1) / tile_rows) * ((columns + tile_columns - 1) / tile_columns);
     };
     const uint64_t wave = (uint64_t)cus;
-    if (rows <= 64u || (rows <= 256u && inner >= 2048u)) {
+    // K = 4096, N = 1024, us: 375 rows 17.0 on two rounds of the 32 x 32
+    // small-M tile, 19.5 on 64 x 64, 22.1 on 96 x 64; 512 rows 18.7, 19.6 and
+    // 22.6; 640 rows 28.1, 19.6 and 22.3.
+    if (rows <= 64u || tiles(32, 32) <= (inner >= 2048u ? 2u * wave : wave)) {
       const int v = find_variant(PK_PRECISION_F16, pk::kFamilySmallM, 1, 1, 1, 1, 8);
       return {v < 0 ? 0 : v, 1u};
     }
-    if (rows <= 256u) {
-      if (columns <= 1024u) {
-        const int v = find_variant(PK_PRECISION_F16, pk::kFamilySmallM, 1, 1, 1, 1, 8);
-        if (v >= 0) return {v, 1u};
-      }
-      return {pair_variant(1, 2, 2, 4), 1u};
+    if (rows <= 256u) return {pair_variant(1, 2, 2, 4), 1u};
+    if (inner >= 2048u) {
+      if (tiles(64, 64) <= wave) return {pair_variant(1, 2, 2, 4), 1u};
+      return {tiles(96, 64) <= wave ? pair_variant(1, 3, 2, 4) : pair_variant(2, 3, 2, 2), 1u};
     }
-    if (inner >= 2048u) return {tiles(96, 64) <= wave ? pair_variant(1, 3, 2, 4) : pair_variant(2, 3, 2, 2), 1u};
     // K <= 256 (the subsampling pointwise convolutions, K = N = 256 over
     // tens of thousands of rows): a workgroup's fixed costs outweigh its K
     // loop, so the K = 1024 figures below mislead. Measured on one MI355X:
@@ -347,7 +348,7 @@ Plan plan_launch(int precision, uint32_t rows, uint32_t inner, uint32_t columns,
     // K < 2048: the fewest rounds of workgroups times the measured time of one
     // workgroup of each tile at K = 1024 with one workgroup per compute unit.
     struct Candidate {
-      int wn, r, c, ks;  // pair-code shape; wn = 0 marks the small-M RW = 2 kernel
+      int wn, r, c, ks;  // pair-code shape
       int tile_rows, tile_columns;
       double us;
     };
@@ -365,7 +366,7 @@ Plan plan_launch(int precision, uint32_t rows, uint32_t inner, uint32_t columns,
     // interleaved on one box; pass 7.13 against 7.16 ms).
     constexpr Candidate kCandidates[] = {
         {2, 6, 2, 2, 192, 128, 22.3}, {2, 4, 2, 2, 128, 128, 17.2}, {2, 3, 2, 2, 96, 128, 14.8},
-        {1, 3, 2, 4, 96, 64, 11.0},   {1, 2, 2, 4, 64, 64, 9.3},    {0, 2, 1, 8, 64, 32, 8.2},
+        {1, 3, 2, 4, 96, 64, 11.0},   {1, 2, 2, 4, 64, 64, 9.3},
         {4, 6, 2, 1, 192, 256, 28.5}, {4, 5, 2, 1, 160, 256, 26.8},
     };
     int best = -1;
@@ -373,8 +374,7 @@ Plan plan_launch(int precision, uint32_t rows, uint32_t inner, uint32_t columns,
     for (const Candidate& c : kCandidates) {
       if (c.tile_columns == 256 && (columns < 3072u || inner < 1024u)) continue;
       if (c.tile_columns == 256 && c.tile_rows == 160 && columns < 3072u) continue;
-      const int v = c.wn ? find_variant(PK_PRECISION_F16, pk::kFamilyPairCode, 1, c.wn, c.r, c.c, c.ks)
-                         : find_variant(PK_PRECISION_F16, pk::kFamilySmallM, 1, 1, c.r, 1, 8);
+      const int v = find_variant(PK_PRECISION_F16, pk::kFamilyPairCode, 1, c.wn, c.r, c.c, c.ks);
       if (v < 0) continue;
       const double rounds = (double)((tiles(c.tile_rows, c.tile_columns) + wave - 1) / wave);
       if (rounds * c.us < best_us * 0.98) {

@@ -42,11 +42,14 @@ using namespace f16;
 // LDS of a variant: the W partial tiles, which during the K loop hold the
 // pair table of a one-palette item instead, and the palettes of up to
 // CB * 32 / 16 + 2 groups of 64 entries.
-template <int W, int RW, int CB>
+template <int W, int RW, int CB, bool STAGED = false>
 struct SmallMShared {
   union {
     float4 red[W * CB * RW * 4 * 64];
-    uint32_t pairs[64 * 64];
+    struct {
+      uint32_t pairs[64 * 64];
+      half8 rows[STAGED ? W : 1][STAGED ? 32 * 8 : 1];  // one K block of 32 rows per wavefront
+    };
   };
   _Float16 lut[(CB * 2 + 2) * 64];
 };
@@ -85,9 +88,10 @@ __device__ __forceinline__ half8 decode_pairs(const uint32_t (&w)[BITS], int s, 
 // GENERAL: the columns may span several palette groups (per-lane palette
 // base) or K may be 32 (mod 64) (the upper half of the last K block is
 // padding: its activation fragments are zeroed).
-template <int BITS, int W, int RW, int CB, int D, bool GENERAL>
+template <int BITS, int W, int RW, int CB, int D, bool GENERAL, bool STAGED>
 __device__ __forceinline__ void small_m_item(const GemmArgs& args, uint32_t cg, uint32_t mg,
-                                             SmallMShared<W, RW, CB>& sh) {
+                                             SmallMShared<W, RW, CB, STAGED>& sh) {
+  static_assert(!STAGED || (RW == 1 && CB == 1 && !GENERAL), "staged rows: 32 x 32 tiles, K % 64 == 0");
   constexpr int T = 64 * W;
   constexpr int E = 1 << BITS;
   constexpr uint32_t BW = block_words(BITS);
@@ -179,11 +183,53 @@ __device__ __forceinline__ void small_m_item(const GemmArgs& args, uint32_t cg, 
 #pragma unroll
       for (int s = 0; s < 4; ++s) dst[mi][s] = *reinterpret_cast<const half8*>(a_row[mi] + k0 + 8u * s);
   };
+  // Staged rows: loaded as fragments, the 64 lanes of a load touch 32 rows,
+  // and the eight wavefronts' rows overflow the L1 between the four loads
+  // that share their lines. So each wavefront loads its block as whole
+  // 128-byte rows, eight lines per load and D blocks ahead, and turns them
+  // into fragments through 4 KB of LDS of its own (its LDS operations
+  // complete in order: no barrier, one buffer). 16-byte chunk c of row r lies
+  // at c ^ (r >> 1) & 7.
+  constexpr int AD = STAGED ? D : 1;
+  half8 ag[AD][4];
+  auto load_rows = [&](uint32_t kb, half8 (&dst)[4]) {
+    const uint32_t chunk = (uint32_t)lane & 7u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t m = min(m0 + (uint32_t)(8 * i + (lane >> 3)), M - 1u);
+      dst[i] = *reinterpret_cast<const half8*>(static_cast<const _Float16*>(args.a) + (uint64_t)m * K + kb * 64u +
+                                               chunk * 8u);
+    }
+  };
+  auto turn_rows = [&](const half8 (&src)[4], half8 (&dst)[RW][4]) {
+    if constexpr (STAGED) {
+      half8* rows = sh.rows[wave];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 8 * i + (lane >> 3);
+        rows[r * 8 + ((lane & 7) ^ ((r >> 1) & 7))] = src[i];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int s = 0; s < 4; ++s) dst[0][s] = rows[j * 8 + ((4 * h + s) ^ ((j >> 1) & 7))];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+  };
   uint32_t cr[D][CB][BITS];
   half8 ar[2][RW][4];
+  if constexpr (STAGED) {
 #pragma unroll
-  for (int d = 0; d < D; ++d) load_codes(block(d), cr[d]);
-  load_a(block(0), ar[0]);
+    for (int d = 0; d < D; ++d) {
+      load_rows(block(d), ag[d]);
+      load_codes(block(d), cr[d]);
+    }
+  } else {
+#pragma unroll
+    for (int d = 0; d < D; ++d) load_codes(block(d), cr[d]);
+    load_a(block(0), ar[0]);
+  }
 
 #pragma unroll
   for (int p = 0; p < PPT; ++p)
@@ -229,13 +275,23 @@ __device__ __forceinline__ void small_m_item(const GemmArgs& args, uint32_t cg, 
 
   __syncthreads();  // palettes (and pair table) staged
   // Whole groups of D blocks, then the last nblocks % D (their codes are
-  // already loaded).
+  // already loaded). The next block's fragments are fetched before each
+  // block's products.
+  if constexpr (STAGED) {
+    turn_rows(ag[0], ar[0]);
+    load_rows(block((uint32_t)AD), ag[0]);
+  }
   uint32_t t = 0;
   for (; t + (uint32_t)D <= nblocks; t += D) {
 #pragma unroll
     for (int u = 0; u < D; ++u) {
       const uint32_t i = t + (uint32_t)u;
-      load_a(block(i + 1u), ar[(u + 1) & 1]);
+      if constexpr (STAGED) {
+        turn_rows(ag[(u + 1) % AD], ar[(u + 1) & 1]);
+        load_rows(block(i + 1u + (uint32_t)AD), ag[(u + 1) % AD]);
+      } else {
+        load_a(block(i + 1u), ar[(u + 1) & 1]);
+      }
       multiply(cr[u], ar[u & 1], block(i));
       load_codes(block(i + (uint32_t)D), cr[u]);
     }
@@ -243,12 +299,15 @@ __device__ __forceinline__ void small_m_item(const GemmArgs& args, uint32_t cg, 
 #pragma unroll
   for (int u = 0; u < D - 1; ++u) {
     if (t + (uint32_t)u < nblocks) {
-      load_a(block(t + (uint32_t)u + 1u), ar[(u + 1) & 1]);
+      if constexpr (STAGED)
+        turn_rows(ag[(u + 1) % AD], ar[(u + 1) & 1]);
+      else
+        load_a(block(t + (uint32_t)u + 1u), ar[(u + 1) & 1]);
       multiply(cr[u], ar[u & 1], block(t + (uint32_t)u));
     }
   }
 
-  if constexpr (!GENERAL) __syncthreads();  // the partials overwrite the pair table
+  if constexpr (!GENERAL) __syncthreads();  // the partials overwrite the pair table and the rows
   // Partials: [wave][tile][quad q][slot] float4, tile = c * RW + mi,
   // slot = lane ^ 2(2q + h), which keeps both the per-lane writes and the
   // row-wise reads on distinct bank groups.
@@ -328,14 +387,14 @@ __device__ __forceinline__ bool small_m_work(uint32_t column_groups, uint32_t ro
   return small_m_work_of(blockIdx.x, column_groups, row_groups, cg, mg);
 }
 
-template <int BITS, int W, int RW, int CB, int D, bool GENERAL>
+template <int BITS, int W, int RW, int CB, int D, bool GENERAL, bool STAGED>
 __global__ __launch_bounds__(64 * W) void gemm_f16s_kernel(GemmArgs args) {
-  __shared__ SmallMShared<W, RW, CB> sh;
+  __shared__ SmallMShared<W, RW, CB, STAGED> sh;
   const uint32_t ncg = ((args.columns + 31u) / 32u + CB - 1u) / CB;
   const uint32_t tm = (args.rows + RW * 32u - 1u) / (RW * 32u);
   uint32_t cg, mg;
   if (!small_m_work(ncg, tm, cg, mg)) return;
-  small_m_item<BITS, W, RW, CB, D, GENERAL>(args, cg, mg, sh);
+  small_m_item<BITS, W, RW, CB, D, GENERAL, STAGED>(args, cg, mg, sh);
 }
 
 // A group: item i of the column-group table names member items[i] >> 16 and
@@ -356,14 +415,14 @@ __global__ __launch_bounds__(64 * W) void gemm_f16s_group_kernel(SmallMGroupArgs
                        (args.palette_groups > 1u && args.palette_group_columns % (uint32_t)(CB * 32) != 0u);
   if (member.bits == 5) {
     if (general)
-      small_m_item<5, W, RW, CB, D, true>(args, cg, mg, sh);
+      small_m_item<5, W, RW, CB, D, true, false>(args, cg, mg, sh);
     else
-      small_m_item<5, W, RW, CB, D, false>(args, cg, mg, sh);
+      small_m_item<5, W, RW, CB, D, false, false>(args, cg, mg, sh);
   } else {
     if (general)
-      small_m_item<6, W, RW, CB, D, true>(args, cg, mg, sh);
+      small_m_item<6, W, RW, CB, D, true, false>(args, cg, mg, sh);
     else
-      small_m_item<6, W, RW, CB, D, false>(args, cg, mg, sh);
+      small_m_item<6, W, RW, CB, D, false, false>(args, cg, mg, sh);
   }
 }
 
@@ -696,8 +755,8 @@ struct SmallMVariant {
   F16Variant {                                                                                             \
     TileShape{1, 1, RW, CB, W}, "pk_gemm_f16s_b5_k" #W "_m" #RW "n" #CB "d" #D,                           \
         "pk_gemm_f16s_b6_k" #W "_m" #RW "n" #CB "d" #D,                                                    \
-        {gemm_f16s_kernel<5, W, RW, CB, D, false>, gemm_f16s_kernel<6, W, RW, CB, D, false>},               \
-        {gemm_f16s_kernel<5, W, RW, CB, D, true>, gemm_f16s_kernel<6, W, RW, CB, D, true>},                 \
+        {gemm_f16s_kernel<5, W, RW, CB, D, false, false>, gemm_f16s_kernel<6, W, RW, CB, D, false, false>}, \
+        {gemm_f16s_kernel<5, W, RW, CB, D, true, false>, gemm_f16s_kernel<6, W, RW, CB, D, true, false>},   \
         (uint32_t)sizeof(SmallMShared<W, RW, CB>)                                                          \
   }
 #define PK_F16S_VARIANT(W, RW, CB, D)                                                                      \
@@ -768,7 +827,14 @@ hipError_t launch_gemm_f16s(int bits, const f16::F16Variant& v, const GemmArgs& 
   if (cgs == 0 || args.rows == 0) return hipSuccess;
   const bool single = (args.inner & 63u) == 0u &&
                       (args.palette_groups == 1 || args.palette_group_columns % (uint32_t)v.shape.tile_columns() == 0);
-  return launch_timed(single ? v.single[bits == 6] : v.general[bits == 6],
+  void (*kernel)(GemmArgs) = single ? v.single[bits == 6] : v.general[bits == 6];
+  // More than one row group of the 32 x 32 tile: the rows come through LDS
+  // (same sums). 188 x 4096 -> 1024 12.1 -> 9.6 us, 64 x 4096 -> 1024 11.3 ->
+  // 8.8, 188 x 1024 -> 1024 6.1 -> 5.7; with one row group (16 rows) the turn
+  // costs more than it saves, 5.0 against 5.2 us for 1024 -> 4096.
+  if (single && args.rows > 32u && v.shape.m_blocks == 1 && v.shape.n_blocks == 1 && v.shape.k_split == 8)
+    kernel = bits == 6 ? gemm_f16s_kernel<6, 8, 1, 1, 4, false, true> : gemm_f16s_kernel<5, 8, 1, 1, 4, false, true>;
+  return launch_timed(kernel,
                       dim3(small_m_grid(v.shape, cgs, args.rows)), dim3(v.shape.threads()), stream, start, stop, args);
 }
 
