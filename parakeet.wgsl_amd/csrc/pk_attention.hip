@@ -97,14 +97,43 @@ __global__ __launch_bounds__(64 * KSPLIT) void rel_attention_f16_kernel(AttnArgs
     return;
   }
 
+  // A key tile's rows, all loads before any use, the next tile's as soon as
+  // the products have read this one's (clamped, unconditional): with one
+  // wavefront per SIMD only these loads overlap the softmax and the PV
+  // products. 256 VGPRs + 230 AGPRs; 1 x 188 12.2 -> 11.8 us, 5 x 188 14.9 ->
+  // 13.5, 1 x 750 33.9 -> 26.7 (1 x 100, one tile per wavefront, 9.1 -> 9.3). The
+  // first tile's loads ahead of the query operands as well: 12.1, 1 x 60 9.3
+  // against 7.6.
+  const int tiles = (live + kTile - 1) / kTile;
+  half8 kv[8], ra[8], rb[8], vx[8];
+  auto load_tile = [&](int kt) {
+    const int k0 = kt * kTile;
+    const int p_lo = T - 1 - q0 - (kTile - 1) + k0;
+    const int pmax = (int)args.position_rows - 1;
+    const _Float16* krow = qkv + (uint64_t)min(k0 + j, T - 1) * kQkvRow + kHidden;
+    const int pa = min(max(p_lo + j, 0), pmax), pb = min(max(p_lo + kTile + j, 0), pmax);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int d0 = 16 * s + 8 * hh;
+      kv[s] = load8(krow + d0);
+      ra[s] = load_position<ROW_MAJOR>(static_cast<const _Float16*>(args.positions), args.position_rows, head, pa, d0);
+      rb[s] = load_position<ROW_MAJOR>(static_cast<const _Float16*>(args.positions), args.position_rows, head, pb, d0);
+    }
+#pragma unroll
+    for (int c = 0; c < 8; ++c) vx[c] = load8(krow + kHidden + 16 * c + 8 * hh);
+  };
+
   // (Q+u)^T and (Q+v)^T operands of query q0 + j: channels 16s + 8hh + 0..7.
   half8 qu[8], qv[8];
   {
     const _Float16* qrow = qkv + (uint64_t)min(q0 + j, T - 1) * kQkvRow;
+    half8 xq[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) xq[s] = load8(qrow + 16 * s + 8 * hh);
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
       const int d0 = 16 * s + 8 * hh;
-      const half8 x = load8(qrow + d0);
+      const half8 x = xq[s];
       const float4 u0 = *reinterpret_cast<const float4*>(args.bias_u + head * kHead + d0);
       const float4 u1 = *reinterpret_cast<const float4*>(args.bias_u + head * kHead + d0 + 4);
       const float4 v0 = *reinterpret_cast<const float4*>(args.bias_v + head * kHead + d0);
@@ -130,41 +159,30 @@ __global__ __launch_bounds__(64 * KSPLIT) void rel_attention_f16_kernel(AttnArgs
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[db][r] = 0.0f;
 
-  const int tiles = (live + kTile - 1) / kTile;
+  load_tile(min(wave, tiles - 1));
   for (int kt = wave; kt < tiles; kt += KSPLIT) {
     const int k0 = kt * kTile;
-    const int p_lo = T - 1 - q0 - (kTile - 1) + k0;
-    const int pmax = (int)args.position_rows - 1;
     // S^T = K (Q+u)^T and W^T = R[p_lo ..] (Q+v)^T.
     floatx16 ac, w0, w1;
 #pragma unroll
     for (int r = 0; r < 16; ++r) ac[r] = w0[r] = w1[r] = 0.0f;
-    const _Float16* krow = qkv + (uint64_t)min(k0 + j, T - 1) * kQkvRow + kHidden;
-    const int pa = min(max(p_lo + j, 0), pmax), pb = min(max(p_lo + kTile + j, 0), pmax);
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
-      const int d0 = 16 * s + 8 * hh;
-      const half8 kv = load8(krow + d0);
-      const half8 ra = load_position<ROW_MAJOR>(static_cast<const _Float16*>(args.positions), args.position_rows,
-                                                head, pa, d0);
-      const half8 rb = load_position<ROW_MAJOR>(static_cast<const _Float16*>(args.positions), args.position_rows,
-                                                head, pb, d0);
-      ac = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv, qu[s], ac, 0, 0, 0);
-      w0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ra, qv[s], w0, 0, 0, 0);
-      w1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(rb, qv[s], w1, 0, 0, 0);
+      ac = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv[s], qu[s], ac, 0, 0, 0);
+      w0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ra[s], qv[s], w0, 0, 0, 0);
+      w1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(rb[s], qv[s], w1, 0, 0, 0);
     }
     // V tile -> LDS, transposed: vt[d][swap23(key)].
     {
-      const _Float16* vrow = qkv + (uint64_t)min(k0 + j, T - 1) * kQkvRow + 2 * kHidden;
       const int slot = (j & ~12) | ((j & 4) << 1) | ((j & 8) >> 1);
 #pragma unroll
       for (int c = 0; c < 8; ++c) {
         const int d0 = 16 * c + 8 * hh;
-        const half8 x = load8(vrow + d0);
 #pragma unroll
-        for (int t = 0; t < 8; ++t) vt[(d0 + t) * kVtStride + slot] = x[t];
+        for (int t = 0; t < 8; ++t) vt[(d0 + t) * kVtStride + slot] = vx[c][t];
       }
     }
+    if (kt + KSPLIT < tiles) load_tile(kt + KSPLIT);
     // Window rows c = 32 blk + 8 (r/4) + 4 hh + r%4, column j.
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
@@ -865,9 +883,11 @@ struct AttnVariant {
 // index 1); index 4 below 1152 (12 / 16 windows: 19.1 / 19.6 us); index 3
 // from 1152 (24 windows: 32.4 against 33.5 us; 40 windows: 39.5 against
 // 51.3 us, where index 4's half-empty second query block per window and
-// head costs more than its shared staging saves); index 4 for windows
-// longer than 256 frames (4 x 750: 46.2 us against 50.6 us for index 3 and
-// 86.9 us for index 0).
+// head costs more than its shared staging saves). For windows longer than 256
+// frames index 0 up to 256 tiles too (1 x 300 14.7 us against 21.9 for index
+// 3 and 24.0 for index 4; 2 x 400 19.7, 27.0, 29.4; 1 x 750 26.7, 44.1, 46.6),
+// index 3 up to 384 (2 x 750 44.6 against 47.3 and 49.7 for index 0) and
+// index 4 beyond (4 x 750: 46.2 us against 50.6 us for index 3).
 const AttnVariant kF16Variants[] = {PK_ATTN_VARIANT(4), PK_ATTN_VARIANT(2), PK_ATTN_VARIANT(1),
                                     PK_ATTN_SHARED_VARIANT(2), PK_ATTN_SHARED_VARIANT(4)};
 // f32: index 0 the MFMA kernel (planned), index 1 one workgroup per query in
@@ -882,9 +902,8 @@ const AttnVariant kF32Variants[] = {
 
 int attention_default_variant(bool f16, uint32_t frames, uint32_t batch) {
   if (!f16) return 0;
-  if (frames > 256u) return 4;
   const uint64_t tiles = (uint64_t)batch * kHeads * ((frames + kTile - 1) / kTile);
-  return tiles <= 256u ? 0 : tiles <= 384u ? 3 : tiles < 1152u ? 4 : 3;
+  return tiles <= 256u ? 0 : tiles <= 384u ? 3 : tiles < 1152u || frames > 256u ? 4 : 3;
 }
 
 int attention_variant_count(bool f16) {
