@@ -400,17 +400,17 @@ Plan plan_launch(int precision, uint32_t rows, uint32_t inner, uint32_t columns,
   // 1024 of K the time of a first workgroup on a compute unit and of each
   // further one, as fitted to a sweep of every tile over 16 to 3008 rows of
   // the encoder's GEMMs (within 15%). What it has to tell apart (us): 3008 x
-  // 1024 -> 4096 122 on 64 x 256 against 131 on 128 x 128 and 136 on 96 x 128;
-  // 3008 x 1024 -> 1024 39.1 on 96 x 128 against 42.5 and 43.4 on 32 and
-  // 64 x 128; 1504 x 1024 -> 1024 25.7 on 64 x 128 against 28.7 and 33.3;
+  // 1024 -> 4096 130 on 64 x 256 against 141 on 96 x 128 and 148 on 64 x 128;
+  // 3008 x 1024 -> 1024 41.4 on 96 x 128 against 44.6 and 45.4 on 32 and
+  // 64 x 128; 1504 x 1024 -> 1024 28.9 on 64 x 128 against 29.1 and 36.4;
   // 188 x 1024 -> 4096 21.3 on 32 x 128 against 23.1 with K over four waves,
-  // which takes 188 x 4096 -> 1024 in 29.6 against 69.2.
+  // which takes 188 x 4096 -> 1024 in 28 against 72.
   struct Tile {
     int wn, mb, nb, ks;
     double first, each;
   };
   constexpr Tile kTiles[] = {{4, 1, 1, 1, 16.0, 14.0}, {4, 2, 1, 1, 20.5, 22.0}, {4, 3, 1, 1, 29.0, 32.0},
-                             {4, 4, 1, 1, 36.0, 43.0}, {4, 2, 2, 1, 34.5, 39.5}, {1, 1, 1, 4, 5.9, 5.9}};
+                             {4, 2, 2, 1, 34.5, 39.5}, {1, 1, 1, 4, 5.9, 5.9}};
   const int count = pk::f32_variant_count();
   int best = 0;
   double best_cost = 1e300;

@@ -6,10 +6,13 @@
 // operand is split into three bf16 terms that add up to it exactly, and six
 // of the nine products of terms go through v_mfma_f32_32x32x16_bf16 into one
 // f32 accumulator, smallest first; the three left out are below 2^-24 of the
-// product. One accumulator addition per 16 k instead of one per 2 k leaves the
-// sums nearer to 64 bits than the f32 units' (norm-wise 4.9e-7 against 5.7e-7
-// at K = 1024, 1.0e-6 against 1.1e-6 at K = 4096, 2.4e-7 and 5.0e-7 with K over
-// four waves).
+// product. The sums are nearer to 64 bits than the f32 units' (norm-wise
+// 4.8e-7 against 5.7e-7 at K = 1024, 9.7e-7 against 1.1e-6 at K = 4096, 2.4e-7
+// and 4.9e-7 with K over four waves). The unit rounds its sums down, though,
+// and half of that error was one offset for all outputs, which attention's
+// average over the keys keeps while it averages the rest away (context of 4 x
+// 253 frames 9.1e-7 against 7.3e-7 before); with every second run of K blocks
+// subtracted the offset is gone (6.2e-7) at 4-6% of the time.
 //
 // Bound: the bf16 matrix units in principle (a sixth of their rate: 417
 // TFLOP/s nominal, about 190 at the rate of a large library product), LDS
@@ -22,8 +25,8 @@
 // gather per code and three byte permutes per pair.
 //
 // Against v_mfma_f32_32x32x2_f32 before: 3008 x 1024 -> 4096 (5-bit) 214 ->
-// 122 us (206 TFLOP/s), 3008 x 4096 -> 1024 227 -> 135, 3008 x 1024 -> 3072 168
-// -> 99, 256 x 1024 -> 4096 (6-bit) 30.5 -> 22.5, 188 x 4096 -> 1024 102 -> 30,
+// 130 us (194 TFLOP/s), 3008 x 4096 -> 1024 227 -> 143, 3008 x 1024 -> 3072 168
+// -> 102, 256 x 1024 -> 4096 (6-bit) 30.5 -> 21.7, 188 x 4096 -> 1024 102 -> 28,
 // 16 x 1024 -> 4096 28 -> 10.
 //
 // Codes in operand order: lane half h owns k = 64 kb + 32 h + u, so MFMA
@@ -93,7 +96,7 @@ __global__ __launch_bounds__(64 * WN * KS, 2) void gemm_f32_kernel(GemmArgs args
   static_assert(BM * 8 % GT == 0, "the A tile divides evenly");
 
   __shared__ __align__(16) uint8_t a_lds_all[KS][3][3 * PLANE];
-  __shared__ uint2 lut_lds[LUT_CAP];  // {hi | mid << 16, lo}
+  __shared__ uint2 lut_lds[2 * LUT_CAP];  // {hi | mid << 16, lo}, then the same negated
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -198,7 +201,9 @@ __global__ __launch_bounds__(64 * WN * KS, 2) void gemm_f32_kernel(GemmArgs args
     const uint32_t entries = (g_hi - g_lo + 1u) * E;
     for (uint32_t i = tid; i < entries; i += T) {
       const Split s = split2(palette[(uint64_t)g_lo * E + i], 0.0f);
-      lut_lds[i] = make_uint2((s.hi & 0xffffu) | s.mid << 16, s.lo & 0xffffu);
+      const uint2 e = make_uint2((s.hi & 0xffffu) | s.mid << 16, s.lo & 0xffffu);
+      lut_lds[i] = e;
+      lut_lds[LUT_CAP + i] = make_uint2(e.x ^ 0x80008000u, e.y ^ 0x8000u);
     }
   }
   uint32_t lut_base[NB];  // first entry of the lane's column's palette group
@@ -209,11 +214,11 @@ __global__ __launch_bounds__(64 * WN * KS, 2) void gemm_f32_kernel(GemmArgs args
   }
   // Weights of a sub-step: the entries of its eight codes per column block,
   // then the three operands.
-  auto gather = [&](const uint32_t (&c)[NB][BITS], int sub, uint2 (&e)[NB][8]) {
+  auto gather = [&](const uint32_t (&c)[NB][BITS], int sub, uint32_t sign, uint2 (&e)[NB][8]) {
 #pragma unroll
     for (int ni = 0; ni < NB; ++ni)
 #pragma unroll
-      for (int u = 0; u < 8; ++u) e[ni][u] = lut_lds[lut_base[ni] + lane_code<BITS>(c[ni], sub * 8 + u)];
+      for (int u = 0; u < 8; ++u) e[ni][u] = lut_lds[lut_base[ni] + sign + lane_code<BITS>(c[ni], sub * 8 + u)];
   };
   auto assemble = [&](const uint2 (&e)[NB][8], bf16x8 (&w)[NB][3]) {
 #pragma unroll
@@ -277,24 +282,39 @@ __global__ __launch_bounds__(64 * WN * KS, 2) void gemm_f32_kernel(GemmArgs args
     bf16x8 w[NB][3], a0[MB][3], a1[MB][3];
     uint2 e[NB][8];
     uint32_t buf = 0;
-    gather(cw, 0, e);
+    gather(cw, 0, 0u, e);
     read_a(0, 0, a0);
     assemble(e, w);
+    // The matrix unit rounds its sums down, not to nearest: a bias that the
+    // average over many outputs (attention over its keys) would show whole.
+    // So every second run of blocks (two, or one of a K part) is subtracted:
+    // negated weights into the negated sum, whose roundings then go up.
+    constexpr uint32_t kRun = KS == 1 ? 2u : 1u;
+    auto sign_of = [&](uint32_t i) { return (i / kRun & 1u) * (uint32_t)LUT_CAP; };
+    auto negate = [&] {
+#pragma unroll
+      for (int mi = 0; mi < MB; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < NB; ++ni)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) acc[mi][ni][v] = -acc[mi][ni][v];
+    };
     for (uint32_t i = 0; i < own_blocks; ++i) {
+      const uint32_t sign = sign_of(i), next_sign = sign_of(i + 1u);
       uint32_t cn[NB][BITS];
       load_codes(min(i + 1u, own_blocks - 1u) * KS + part, cn);
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
         const uint32_t t = 2u * i + half;
         const uint32_t buf1 = buf == 2u ? 0u : buf + 1u, buf2 = buf1 == 2u ? 0u : buf1 + 1u;
-        gather(cw, 2 * half + 1, e);
+        gather(cw, 2 * half + 1, sign, e);
         read_a(buf, 1, a1);
         multiply(w, a0);
         assemble(e, w);
         if (half == 0)
-          gather(cw, 2, e);
+          gather(cw, 2, sign, e);
         else
-          gather(cn, 0, e);
+          gather(cn, 0, next_sign, e);
         read_a(buf1, 0, a0);
         store_a(min(t + 2u, steps - 1u), buf2, a_stage[half]);
         load_a(min(t + 4u, steps - 1u), a_stage[half]);
@@ -307,6 +327,7 @@ __global__ __launch_bounds__(64 * WN * KS, 2) void gemm_f32_kernel(GemmArgs args
       for (int ni = 0; ni < NB; ++ni)
 #pragma unroll
         for (int q = 0; q < BITS; ++q) cw[ni][q] = cn[ni][q];
+      if (i + 1u < own_blocks ? sign != next_sign : sign != 0u) negate();
     }
   }
 
@@ -442,7 +463,6 @@ const Variant kVariants[] = {
     PK_F32_VARIANT(4, 1, 1, 1),  // 32 x 128
     PK_F32_VARIANT(4, 2, 1, 1),  // 64 x 128
     PK_F32_VARIANT(4, 3, 1, 1),  // 96 x 128
-    PK_F32_VARIANT(4, 4, 1, 1),  // 128 x 128
     PK_F32_VARIANT(4, 2, 2, 1),  // 64 x 256
     PK_F32_VARIANT(1, 1, 1, 4),  // 32 x 32, K over four waves
 };
