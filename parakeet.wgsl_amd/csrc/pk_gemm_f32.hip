@@ -6,7 +6,12 @@
 // operand is split into three bf16 terms that add up to it exactly, and six
 // of the nine products of terms go through v_mfma_f32_32x32x16_bf16 into one
 // f32 accumulator, smallest first; the three left out are below 2^-24 of the
-// product. The sums are nearer to 64 bits than the f32 units' (norm-wise
+// product. bf16 has the exponents of f32 but not the 16 bits below them that
+// the second and third term of an operand under 2^-110 need, so both operands
+// are multiplied by 2^24 before the split and the sum by 2^-48 after it:
+// every term down to the last bit of the smallest subnormal f32 is then a
+// normal bf16. Operands from 2^104 and sums from 2^80 on overflow instead and
+// come from the f32 units, output by output. The sums are nearer to 64 bits than the f32 units' (norm-wise
 // 4.8e-7 against 5.7e-7 at K = 1024, 9.7e-7 against 1.1e-6 at K = 4096, 2.4e-7
 // and 4.9e-7 with K over four waves). The unit rounds its sums down, though,
 // and half of that error was one offset for all outputs, which attention's
@@ -68,8 +73,11 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
 __device__ __forceinline__ float low_f32(uint32_t p) { return __uint_as_float(p << 16); }
 __device__ __forceinline__ float high_f32(uint32_t p) { return __uint_as_float(p & 0xffff0000u); }
 
-// Two f32 values as three bf16 terms each, rounded to nearest one after the
-// other: the sum of the three is the value (8 + 8 + 8 significand bits).
+constexpr float kOperandScale = 0x1p24f, kSumScale = 0x1p-48f;
+
+// Two scaled f32 values as three bf16 terms each, rounded to nearest one
+// after the other: the sum of the three is the value (8 + 8 + 8 significand
+// bits, and no term below the smallest normal bf16).
 struct Split {
   uint32_t hi, mid, lo;
 };
@@ -172,10 +180,10 @@ __global__ __launch_bounds__(64 * WN * KS, 2) void gemm_f32_kernel(GemmArgs args
     for (int c = 0; c < CH; ++c) {
       const int idx = gtid + c * GT;
       const int r = idx >> 3, run = idx & 7;
-      const bool inside = run_k(t, run) < K;
+      const float scale = run_k(t, run) < K ? kOperandScale : 0.0f;
       const float4 x = stage[c];
-      const Split s0 = split2(inside ? x.x : 0.0f, inside ? x.y : 0.0f);
-      const Split s1 = split2(inside ? x.z : 0.0f, inside ? x.w : 0.0f);
+      const Split s0 = split2(x.x * scale, x.y * scale);
+      const Split s1 = split2(x.z * scale, x.w * scale);
       const int chunk = ((run >> 1) & 1) * 2 + (run >> 2);
       uint8_t* dst = &a_lds[buf][r * 64 + ((chunk ^ ((r >> 2) & 3)) << 4) + (run & 1) * 8];
       *reinterpret_cast<uint2*>(dst) = make_uint2(s0.hi, s1.hi);
@@ -200,7 +208,7 @@ __global__ __launch_bounds__(64 * WN * KS, 2) void gemm_f32_kernel(GemmArgs args
   {
     const uint32_t entries = (g_hi - g_lo + 1u) * E;
     for (uint32_t i = tid; i < entries; i += T) {
-      const Split s = split2(palette[(uint64_t)g_lo * E + i], 0.0f);
+      const Split s = split2(palette[(uint64_t)g_lo * E + i] * kOperandScale, 0.0f);
       const uint2 e = make_uint2((s.hi & 0xffffu) | s.mid << 16, s.lo & 0xffffu);
       lut_lds[i] = e;
       lut_lds[LUT_CAP + i] = make_uint2(e.x ^ 0x80008000u, e.y ^ 0x8000u);
@@ -315,9 +323,12 @@ __global__ __launch_bounds__(64 * WN * KS, 2) void gemm_f32_kernel(GemmArgs args
           gather(cw, 2, sign, e);
         else
           gather(cn, 0, next_sign, e);
-        read_a(buf1, 0, a0);
+        // three row blocks: the split of the new rows first (3008 x 4096 -> 1024
+        // 143 us against 146; 32 x 128 and 64 x 256 lose 2% and 10% that way)
+        if constexpr (MB < 3) read_a(buf1, 0, a0);
         store_a(min(t + 2u, steps - 1u), buf2, a_stage[half]);
         load_a(min(t + 4u, steps - 1u), a_stage[half]);
+        if constexpr (MB >= 3) read_a(buf1, 0, a0);
         multiply(w, a1);
         assemble(e, w);
         sync();
@@ -331,17 +342,23 @@ __global__ __launch_bounds__(64 * WN * KS, 2) void gemm_f32_kernel(GemmArgs args
     }
   }
 
-  // A value that is infinite, NaN or rounds up past the largest bf16 has no
-  // split: its rows or columns come out as NaN or infinity. A wave that
-  // finds one computes its blocks again on the f32 units, one code and one
-  // element of A per lane and MFMA.
+  // A value that is infinite, NaN or past the largest bf16 once scaled has no
+  // split: its rows or columns come out as NaN or infinity, as a scaled sum
+  // that overflows does. A wave that finds one computes its blocks again on
+  // the f32 units, one code and one element of A per lane and MFMA, and takes
+  // the outputs that are not finite from there: which sum an output gets
+  // depends on its own row and column alone.
+  auto is_finite = [](float x) { return __builtin_fabsf(x) <= 3.402823466e+38f; };
   bool finite = true;
 #pragma unroll
   for (int mi = 0; mi < MB; ++mi)
 #pragma unroll
     for (int ni = 0; ni < NB; ++ni)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) finite &= __builtin_fabsf(acc[mi][ni][v]) <= 3.402823466e+38f;
+      for (int v = 0; v < 16; ++v) {
+        acc[mi][ni][v] *= kSumScale;
+        finite &= is_finite(acc[mi][ni][v]);
+      }
   if (!__all(finite)) {
 #pragma unroll 1
     for (int ni = 0; ni < NB; ++ni) {
@@ -370,7 +387,9 @@ __global__ __launch_bounds__(64 * WN * KS, 2) void gemm_f32_kernel(GemmArgs args
         for (int i = 0; i < MB; ++i)
 #pragma unroll
           for (int o = 0; o < NB; ++o)
-            if (i == mi && o == ni) acc[i][o] = c;
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+              if (i == mi && o == ni && !is_finite(acc[i][o][v])) acc[i][o][v] = c[v];
       }
     }
   }

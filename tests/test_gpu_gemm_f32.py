@@ -95,3 +95,35 @@ def test_sums_have_no_offset(abi, ctx, scope, workloads):
         offset = np.mean(got - want) / np.mean(np.abs(want))
         print("variant", variant, "offset", offset, flush=True)
         assert abs(offset) <= 3.4e-8
+
+
+@pytest.mark.parametrize("exponent", [-100, -112, -120, -126, -140])
+@pytest.mark.parametrize("where", ["a", "palette"])
+def test_operands_down_to_the_smallest_subnormals(abi, ctx, scope, workloads, where, exponent):
+    """Operands of about 2^exponent against ones of about 2^60: the bits that
+    bf16's exponent range has no room for count like any other's."""
+    case = workloads.gemm_case(17, 70, 320, 160, 5, dtype=np.float32)
+    w = case.weight.palette
+    small, large = (case.a, w) if where == "a" else (w, case.a)
+    small[...] = np.ldexp(small.astype(np.float64) / small.std(), exponent).astype(np.float32)
+    large[...] = np.ldexp(large.astype(np.float64) / large.std(), 60).astype(np.float32)
+    want = exact(workloads, case)
+    for variant in range(abi.variant_count("f32")):
+        got = run_case(abi, ctx, scope, case, variant=variant)
+        error = np.linalg.norm(got - want) / np.linalg.norm(want)
+        print(where, exponent, "variant", variant, "error", error, flush=True)
+        assert error <= TOLERANCE
+
+
+def test_an_output_depends_on_its_own_row_and_column_alone(abi, ctx, scope, workloads):
+    """A row that is not finite leaves the other rows of its tile as they are, to the bit."""
+    case = workloads.gemm_case(19, 96, 256, 160, 5, dtype=np.float32)
+    clean = case.a.copy()
+    for variant in range(abi.variant_count("f32")):
+        case.a[...] = clean
+        want = run_case(abi, ctx, scope, case, variant=variant)
+        case.a[[2, 70], 9] = np.nan, 3e38
+        got = run_case(abi, ctx, scope, case, variant=variant)
+        others = np.setdiff1d(np.arange(96), [2, 70])
+        assert np.isnan(got[2]).all()
+        np.testing.assert_array_equal(got[others].view(np.uint32), want[others].view(np.uint32))
