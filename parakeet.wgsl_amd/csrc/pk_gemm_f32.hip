@@ -11,13 +11,14 @@
 // are multiplied by 2^24 before the split and the sum by 2^-48 after it:
 // every term down to the last bit of the smallest subnormal f32 is then a
 // normal bf16. Operands from 2^104 and sums from 2^80 on overflow instead and
-// come from the f32 units, output by output. The sums are nearer to 64 bits than the f32 units' (norm-wise
-// 4.8e-7 against 5.7e-7 at K = 1024, 9.7e-7 against 1.1e-6 at K = 4096, 2.4e-7
-// and 4.9e-7 with K over four waves). The unit rounds its sums down, though,
-// and half of that error was one offset for all outputs, which attention's
-// average over the keys keeps while it averages the rest away (context of 4 x
-// 253 frames 9.1e-7 against 7.3e-7 before); with every second run of K blocks
-// subtracted the offset is gone (6.2e-7) at 4-6% of the time.
+// come from the f32 units, output by output. The sums are nearer to 64 bits
+// than the f32 units' (norm-wise 4.8e-7 against 5.7e-7 at K = 1024, 9.6e-7
+// against 1.1e-6 at K = 4096, 2.4e-7 and 4.8e-7 with K over four waves). The
+// unit rounds its sums down, though, and half of that error was one offset for
+// all outputs, which attention's average over the keys keeps while it averages
+// the rest away (context of 4 x 253 frames 9.1e-7 against 7.3e-7 before); with
+// half of the K blocks subtracted the offset is gone (6.2e-7) at 4-6% of the
+// time.
 //
 // Bound: the bf16 matrix units in principle (a sixth of their rate: 417
 // TFLOP/s nominal, about 190 at the rate of a large library product), LDS
@@ -290,15 +291,24 @@ __global__ __launch_bounds__(64 * WN * KS, 2) void gemm_f32_kernel(GemmArgs args
     bf16x8 w[NB][3], a0[MB][3], a1[MB][3];
     uint2 e[NB][8];
     uint32_t buf = 0;
-    gather(cw, 0, 0u, e);
-    read_a(0, 0, a0);
-    assemble(e, w);
     // The matrix unit rounds its sums down, not to nearest: a bias that the
     // average over many outputs (attention over its keys) would show whole.
-    // So every second run of blocks (two, or one of a K part) is subtracted:
-    // negated weights into the negated sum, whose roundings then go up.
-    constexpr uint32_t kRun = KS == 1 ? 2u : 1u;
-    auto sign_of = [&](uint32_t i) { return (i / kRun & 1u) * (uint32_t)LUT_CAP; };
+    // So half of the runs of blocks (two, or one of a K part or of K <= 128)
+    // are subtracted: negated weights into the negated sum, whose roundings
+    // then go up. The order + - - + - + + - (the parity of the run's bits)
+    // takes out the growth of the sum along K as well, and the K parts begin
+    // with signs in that order. Mean offset, in units of the mean magnitude:
+    // 1e-8 without (K = 128) -> 1.3e-9, K = 1024 -7e-10 (every second run
+    // 4.0e-9, the f32 units -1.0e-9), K = 4096 2.7e-9 (8.1e-9, -2.0e-9). One
+    // block (K <= 64) has nothing to alternate with and keeps -9e-9, a tenth of
+    // its error; changing sign between its halves left -3.5e-9 and cost 64 x
+    // 128 tiles 3% at every K.
+    const uint32_t run_shift = KS == 1 && own_blocks > 2u ? 1u : 0u;
+    const uint32_t first = KS > 1 ? (uint32_t)__popc(__builtin_amdgcn_readfirstlane((int)part)) : 0u;
+    auto sign_of = [&](uint32_t i) { return (((uint32_t)__popc(i >> run_shift) + first) & 1u) * (uint32_t)LUT_CAP; };
+    gather(cw, 0, sign_of(0), e);
+    read_a(0, 0, a0);
+    assemble(e, w);
     auto negate = [&] {
 #pragma unroll
       for (int mi = 0; mi < MB; ++mi)
