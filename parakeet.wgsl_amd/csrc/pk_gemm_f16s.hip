@@ -829,11 +829,14 @@ hipError_t launch_gemm_f16s(int bits, const f16::F16Variant& v, const GemmArgs& 
   const bool single = (args.inner & 63u) == 0u &&
                       (args.palette_groups == 1 || args.palette_group_columns % (uint32_t)v.shape.tile_columns() == 0);
   void (*kernel)(GemmArgs) = single ? v.single[bits == 6] : v.general[bits == 6];
-  // More than one row group of the 32 x 32 tile: the rows come through LDS
-  // (same sums). 188 x 4096 -> 1024 12.1 -> 9.6 us, 64 x 4096 -> 1024 11.3 ->
-  // 8.8, 188 x 1024 -> 1024 6.1 -> 5.7; with one row group (16 rows) the turn
-  // costs more than it saves, 5.0 against 5.2 us for 1024 -> 4096.
-  if (single && args.rows > 32u && v.shape.m_blocks == 1 && v.shape.n_blocks == 1 && v.shape.k_split == 8)
+  // More than one row group of the 32 x 32 tile and K from 768 on: the rows
+  // come through LDS (same sums). 188 x 4096 -> 1024 12.1 -> 9.6 us, 64 x 4096
+  // -> 1024 11.3 -> 8.8, 188 x 1024 -> 1024 6.1 -> 5.5, 64 x 896 -> 1024 5.5 ->
+  // 5.2, 64 x 768 -> 1024 5.0 on both; a wavefront with one K block only fills
+  // its four rows of loads ahead in vain (188 x 512 -> 512 3.9 -> 4.7, 64 x 640
+  // -> 1024 4.6 -> 4.9), and with one row group (16 rows) the turn costs more
+  // than it saves, 5.0 against 5.2 us for 1024 -> 4096.
+  if (single && args.rows > 32u && args.inner >= 768u && v.shape.m_blocks == 1 && v.shape.n_blocks == 1 && v.shape.k_split == 8)
     kernel = bits == 6 ? gemm_f16s_kernel<6, 8, 1, 1, 4, false, true> : gemm_f16s_kernel<5, 8, 1, 1, 4, false, true>;
   return launch_timed(kernel,
                       dim3(small_m_grid(v.shape, cgs, args.rows)), dim3(v.shape.threads()), stream, start, stop, args);

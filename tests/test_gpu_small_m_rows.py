@@ -16,9 +16,11 @@ def scope(ctx):
     s.close()
 
 
-# fewer K blocks than wavefronts, one each, uneven shares, four and more each
+# both forms at their border, uneven shares, four and more K blocks each; and
+# below it, where every row count reads fragments from memory
 @pytest.mark.parametrize("rows,inner,columns,bits,scale", [
-    (33, 64, 32, 5, None), (34, 512, 96, 6, 0.5), (63, 640, 160, 5, None), (64, 1024, 4096, 5, None),
+    (33, 64, 32, 5, None), (34, 512, 96, 6, 0.5), (63, 704, 160, 5, None), (61, 768, 160, 5, None),
+    (90, 832, 64, 6, None), (64, 1024, 4096, 5, None),
     (95, 2112, 64, 6, None), (188, 4096, 1024, 5, 0.5), (300, 2624, 96, 5, None)])
 def test_staged_rows_match_fragments(abi, ctx, scope, oracle, workloads, rows, inner, columns, bits, scale):
     names = variant_names(abi, ctx, scope, workloads)
