@@ -297,12 +297,18 @@ int find_variant(int precision, int family, int waves_m, int waves_n, int m_bloc
 // compiled tile shape over the encoder's GEMM shapes (M 1..3008, K
 // 1024/4096, N 1024..4096, the rel-pos linear's 2T-1 rows). Up to 64 rows,
 // and while its 32 x 32 tiles fit one round of the compute units (two rounds
-// of a deep-K GEMM, K >= 2048), the small-M kernel (32-row blocks, K round
-// robin over eight wavefronts) wins (188 x 1024 -> 1024: 5.7 us against 8.2
-// for the 64 x 64 pair-code tile; 300 x 1024 -> 640 5.4 against 7.9); up to 256
-// rows otherwise the 64 x 64 pair-code tile (188 x 1024 -> 2048 8.0 us against
-// 8.9, -> 4096 8.2 against 12.7); deep-K shapes take 64 x 64 and 96 x 64 while
-// those fill the chip and 96 x 128 beyond. Every other shape takes the
+// from K = 4096 on), the small-M kernel (32-row blocks, K round robin over
+// eight wavefronts) wins (188 x 1024 -> 1024: 5.5 us against 7.8 for the 64 x
+// 64 pair-code tile; 300 x 1024 -> 640 5.5 against 7.8). It deals whole column
+// groups to the eight XCDs, so its rounds are those of the fullest one: two
+// column groups of 1504 rows are 47 tiles on each of two XCDs (1504 x 1024 ->
+// 64 9.3 us against 8.2 for 64 x 64). Below K = 1024 its 64 x 32 tiles win
+// where they make one round and the 32 x 32 ones do not (1024 x 512 -> 512 5.5
+// us against 6.6 for 64 x 64, 1504 x 256 -> 256 5.3 against 5.5, 512 x 768 ->
+// 768 7.3 against 7.5; 512 x 1024 -> 1024 9.2 against 8.4, 600 x 64 -> 512 5.2
+// against 4.9); up to 256 rows otherwise the 64 x 64 pair-code tile (188 x
+// 1024 -> 2048 7.8 us against 8.9, -> 4096 8.2 against 12.7); deep-K shapes
+// take 64 x 64 and 96 x 64 while those fill the chip and 96 x 128 beyond. Every other shape takes the
 // candidate with the least (rounds of workgroups) x (measured time of one
 // workgroup), which puts 192 x 128 on the FF expand and convolution PW1,
 // 96 x 128 on 3000-row 1024-wide GEMMs and 64 x 64 on 752 x 1024 and the
@@ -319,12 +325,23 @@ Plan plan_launch(int precision, uint32_t rows, uint32_t inner, uint32_t columns,
       return (uint64_t)((rows + tile_rows - 1) / tile_rows) * ((columns + tile_columns - 1) / tile_columns);
     };
     const uint64_t wave = (uint64_t)cus;
-    // K = 4096, N = 1024, us: 375 rows 17.0 on two rounds of the 32 x 32
-    // small-M tile, 19.5 on 64 x 64, 22.1 on 96 x 64; 512 rows 18.7, 19.6 and
-    // 22.6; 640 rows 28.1, 19.6 and 22.3.
-    if (rows <= 64u || tiles(32, 32) <= (inner >= 2048u ? 2u * wave : wave)) {
+    // Tiles of the small-M kernel on the XCD that has most, in eighths of the chip.
+    auto small_m_tiles = [&](uint32_t tile_rows) {
+      return 8u * (uint64_t)((rows + tile_rows - 1) / tile_rows) * (((columns + 31u) / 32u + 7u) / 8u);
+    };
+    // K = 4096, N = 1024, us: 375 rows 16.4 on two rounds of the 32 x 32
+    // small-M tile, 19.5 on 64 x 64, 21.9 on 96 x 64; 512 rows 18.6, 19.8 and
+    // 22.7; 600 rows 26.5, 20.4 and 22.9; 1504 rows, N = 256: 22.2 on two
+    // rounds, 20.3 on 64 x 64. K = 2048: 1024 x 512 13.3 and 12.3, 256 x 2048
+    // 12.1 and 11.9.
+    const uint64_t small = small_m_tiles(32u);
+    if (rows <= 64u || small <= wave || (inner >= 4096u && rows <= 1024u && small <= 2u * wave)) {
       const int v = find_variant(PK_PRECISION_F16, pk::kFamilySmallM, 1, 1, 1, 1, 8);
       return {v < 0 ? 0 : v, 1u};
+    }
+    if (inner < 1024u && (inner >= 256u || inner % 64u != 0u) && small_m_tiles(64u) <= wave) {
+      const int v = find_variant(PK_PRECISION_F16, pk::kFamilySmallM, 1, 1, 2, 1, 8);
+      if (v >= 0) return {v, 1u};
     }
     if (rows <= 256u) return {pair_variant(1, 2, 2, 4), 1u};
     if (inner >= 2048u) {
