@@ -421,7 +421,9 @@ Plan plan_launch(int precision, uint32_t rows, uint32_t inner, uint32_t columns,
   // 3008 x 1024 -> 1024 41.4 on 96 x 128 against 44.6 and 45.4 on 32 and
   // 64 x 128; 1504 x 1024 -> 1024 28.9 on 64 x 128 against 29.1 and 36.4;
   // 188 x 1024 -> 4096 21.3 on 32 x 128 against 23.1 with K over four waves,
-  // which takes 188 x 4096 -> 1024 in 28 against 72.
+  // which takes 188 x 4096 -> 1024 in 28 against 72. Each of those waves takes
+  // whole K blocks of 64, so K counts as the next multiple of 256 there (256 x
+  // 64 -> 512: 5.0 us, 4.5 on 32 x 128; 3008 x 128 -> 128 7.2 and 6.2).
   struct Tile {
     int wn, mb, nb, ks;
     double first, each;
@@ -436,7 +438,8 @@ Plan plan_launch(int precision, uint32_t rows, uint32_t inner, uint32_t columns,
     for (const Tile& t : kTiles) {
       if (t.wn != s.waves_n || t.mb != s.m_blocks || t.nb != s.n_blocks || t.ks != s.k_split) continue;
       const double tiles = (double)pk::tiles_m(s, rows) * pk::tiles_n(s, columns);
-      const double cost = 4.5 + (t.first + (std::ceil(tiles / cus) - 1.0) * t.each) * inner / 1024.0;
+      const double k = t.ks > 1 ? std::ceil(inner / (64.0 * t.ks)) * 64.0 * t.ks : (double)inner;
+      const double cost = 4.5 + (t.first + (std::ceil(tiles / cus) - 1.0) * t.each) * k / 1024.0;
       if (cost < best_cost * 0.999) {
         best_cost = cost;
         best = i;
