@@ -173,18 +173,24 @@ __global__ __launch_bounds__(64 * WN * KS, 2) void gemm_f32_kernel(GemmArgs args
       stage[c] = *reinterpret_cast<const float4*>(a_ptr + (uint64_t)m * K + k);
     }
   };
+  auto scale_a = [&](uint32_t t, float4 (&stage)[CH]) {
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const float scale = run_k(t, (gtid + c * GT) & 7) < K ? kOperandScale : 0.0f;
+      stage[c] = make_float4(stage[c].x * scale, stage[c].y * scale, stage[c].z * scale, stage[c].w * scale);
+    }
+  };
   // A row of a term is 64 bytes, chunk 2 s + h of 16 for sub-step s and lane
   // half h; rows four apart start at the same bank, so the chunk is XORed
   // with bits 2 and 3 of the row.
-  auto store_a = [&](uint32_t t, uint32_t buf, const float4 (&stage)[CH]) {
+  auto store_a = [&](uint32_t buf, const float4 (&stage)[CH]) {
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
       const int idx = gtid + c * GT;
       const int r = idx >> 3, run = idx & 7;
-      const float scale = run_k(t, run) < K ? kOperandScale : 0.0f;
       const float4 x = stage[c];
-      const Split s0 = split2(x.x * scale, x.y * scale);
-      const Split s1 = split2(x.z * scale, x.w * scale);
+      const Split s0 = split2(x.x, x.y);
+      const Split s1 = split2(x.z, x.w);
       const int chunk = ((run >> 1) & 1) * 2 + (run >> 2);
       uint8_t* dst = &a_lds[buf][r * 64 + ((chunk ^ ((r >> 2) & 3)) << 4) + (run & 1) * 8];
       *reinterpret_cast<uint2*>(dst) = make_uint2(s0.hi, s1.hi);
@@ -279,9 +285,11 @@ __global__ __launch_bounds__(64 * WN * KS, 2) void gemm_f32_kernel(GemmArgs args
   };
   if constexpr (KS > 1) __syncthreads();  // the palette
   if (steps) {
-    store_a(0, 0, a_stage[0]);
+    scale_a(0, a_stage[0]);
+    scale_a(1, a_stage[1]);
+    store_a(0, a_stage[0]);
     load_a(min(2u, steps - 1u), a_stage[0]);
-    store_a(1, 1, a_stage[1]);
+    store_a(1, a_stage[1]);
     load_a(min(3u, steps - 1u), a_stage[1]);
     sync();
 
@@ -328,6 +336,10 @@ __global__ __launch_bounds__(64 * WN * KS, 2) void gemm_f32_kernel(GemmArgs args
         gather(cw, 2 * half + 1, sign, e);
         read_a(buf, 1, a1);
         multiply(w, a0);
+        // ahead of the split, whose chain a wave alone on its SIMD waits for
+        // (96 x 128, 512 x 4096 -> 1024: 122.7 us, 127.0 inside it)
+        const uint32_t next = min(t + 2u, steps - 1u);
+        scale_a(next, a_stage[half]);
         assemble(e, w);
         if (half == 0)
           gather(cw, 2, sign, e);
@@ -336,7 +348,7 @@ __global__ __launch_bounds__(64 * WN * KS, 2) void gemm_f32_kernel(GemmArgs args
         // three row blocks: the split of the new rows first (3008 x 4096 -> 1024
         // 143 us against 146; 32 x 128 and 64 x 256 lose 2% and 10% that way)
         if constexpr (MB < 3) read_a(buf1, 0, a0);
-        store_a(min(t + 2u, steps - 1u), buf2, a_stage[half]);
+        store_a(buf2, a_stage[half]);
         load_a(min(t + 4u, steps - 1u), a_stage[half]);
         if constexpr (MB >= 3) read_a(buf1, 0, a0);
         multiply(w, a1);
