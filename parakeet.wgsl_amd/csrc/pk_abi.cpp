@@ -253,6 +253,17 @@ int group_width_index(uint32_t column_blocks) {
   return -1;
 }
 
+// LDS of a kernel as it was compiled (0 for none).
+int static_lds(int device, const void* kernel, uint32_t* bytes) {
+  *bytes = 0;
+  if (!kernel) return PK_OK;
+  hipFuncAttributes attributes{};
+  PK_HIP(hipSetDevice(device), "hipSetDevice");
+  PK_HIP(hipFuncGetAttributes(&attributes, kernel), "hipFuncGetAttributes");
+  *bytes = (uint32_t)attributes.sharedSizeBytes;
+  return PK_OK;
+}
+
 // Compulsory HBM bytes of one launch over `rows` rows: the packed codes at
 // the format's density, the palettes, A, the output (+ bias, residual).
 uint64_t algorithmic_bytes(const pk::GemmArgs& a, int bits, uint64_t rows, uint32_t elem) {
@@ -1270,19 +1281,16 @@ int pk_gemm_plan(const pk_gemm_op* op, uint32_t active_rows, pk_gemm_plan_info* 
   info->split_inner = splits;
   info->workspace_bytes = op->workspace_bytes;
   const uint32_t elem = f16 ? 2u : 4u;
-  if (f16) {
-    info->lds_bytes = pk::f16_variant_lds_bytes(variant);
-  } else {
-    const uint32_t lut_cap = (s.tile_columns() / 16u + 2u) * (1u << op->bits);
-    info->lds_bytes = 2u * s.tile_rows() * 256u + lut_cap * elem;
-  }
   info->flops = 2ull * rows * op->args.inner * op->args.columns;
   info->algorithmic_bytes = algorithmic_bytes(op->args, op->bits, rows, elem);
-  std::snprintf(info->kernel, sizeof info->kernel, "%s",
-                f16 ? pk::f16_variant_name(op->bits, variant) : pk::f32_variant_name(op->bits, variant));
   pk::GemmArgs launched = op->args;
   launched.rows = rows;
   launched.stream_out = stream_outputs(op);
+  const char* name = pk::f32_variant_name(op->bits, variant);
+  const pk::GemmKernel kernel =
+      f16 ? pk::f16_kernel(op->bits, variant, launched, &name) : pk::f32_kernel(op->bits, variant);
+  if (int st = static_lds(op->ctx->device, reinterpret_cast<const void*>(kernel), &info->lds_bytes)) return st;
+  std::snprintf(info->kernel, sizeof info->kernel, "%s", name);
   info->stream_stores = f16 && pk::f16_variant_streams(op->bits, variant, launched);
   return ok();
 }
@@ -1487,19 +1495,20 @@ int pk_gemm_group_plan(const pk_gemm_group* g, uint32_t active_rows, pk_gemm_pla
   const pk::TileShape s = pk::f16_variant(variant);
   const int w = group_width_index((uint32_t)s.n_blocks);
   std::memset(info, 0, sizeof *info);
-  const char* kernel = nullptr;
-  info->grid[0] = w < 0 ? 0u : pk::f16_group_launch_plan(variant, group_args(g, variant, rows), &kernel);
+  pk::GemmGroupKernel kernel = nullptr;
+  const char* name = pk::f16_group_kernel_name(variant);
+  info->grid[0] = w < 0 ? 0u : pk::f16_group_launch_plan(variant, group_args(g, variant, rows), &kernel, &name);
   info->grid[1] = info->grid[2] = 1;
   info->block_threads = s.threads();
   info->tile_rows = s.tile_rows();
   info->tile_columns = s.tile_columns();
   info->split_inner = 1;
-  info->lds_bytes = pk::f16_variant_lds_bytes(variant);
+  if (int st = static_lds(g->ctx->device, reinterpret_cast<const void*>(kernel), &info->lds_bytes)) return st;
   for (const pk::SmallMMember& m : g->members) {
     info->flops += 2ull * rows * m.args.inner * m.args.columns;
     info->algorithmic_bytes += algorithmic_bytes(m.args, m.bits, rows, 2u);
   }
-  std::snprintf(info->kernel, sizeof info->kernel, "%s", kernel ? kernel : pk::f16_group_kernel_name(variant));
+  std::snprintf(info->kernel, sizeof info->kernel, "%s", name);
   return ok();
 }
 

@@ -230,7 +230,6 @@ struct F16Variant {
   const char* name6;
   void (*single[2])(GemmArgs);  // [bits == 6]
   void (*general[2])(GemmArgs);
-  uint32_t lds_bytes;           // static LDS of the kernel
   void (*normed[2])(GemmArgs);  // fused row LayerNorm (single path), or null
   void (*streamed[2])(GemmArgs);  // single path with non-temporal output stores, or null
 };
@@ -254,18 +253,16 @@ inline bool streams(const F16Variant& v, int bits, const GemmArgs& a) {
 // Pair-code K-split tile shapes (pk_gemm_f16k.hip).
 int f16k_variant_count();
 const f16::F16Variant& f16k_variant(int index);
-hipError_t launch_gemm_f16k(int bits, const f16::F16Variant& v, const GemmArgs& args, hipStream_t stream,
-                            hipEvent_t start, hipEvent_t stop);
+GemmKernel f16k_kernel(int bits, const f16::F16Variant& v, const GemmArgs& args);
 
 // Small-M shapes (pk_gemm_f16s.hip).
 int f16s_variant_count();
 const f16::F16Variant& f16s_variant(int index);
-hipError_t launch_gemm_f16s(int bits, const f16::F16Variant& v, const GemmArgs& args, hipStream_t stream,
-                            hipEvent_t start, hipEvent_t stop);
+GemmKernel f16s_kernel(int bits, const f16::F16Variant& v, const GemmArgs& args, const char** name);
 const char* f16s_group_name(int index);
 bool f16s_group_persistent(int index);
 bool f16s_group_streams(int index, uint32_t inner, uint32_t palette_groups, uint32_t palette_group_columns);
-uint32_t f16s_group_launch(int index, const SmallMGroupArgs& g, void (**kernel)(SmallMGroupArgs), const char** name);
+uint32_t f16s_group_launch(int index, const SmallMGroupArgs& g, GemmGroupKernel* kernel, const char** name);
 hipError_t launch_gemm_f16s_group(int index, const SmallMGroupArgs& group, hipStream_t stream, hipEvent_t start,
                                   hipEvent_t stop);
 

@@ -283,20 +283,12 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f16_kernel(GemmArgs args) {
   store_tile<WM, WN, R, C, 2 * BM * ROW_BYTES>(args, acc, a_lds, m0, n0, wave_m, wave_n, j, h, tid);
 }
 
-template <int WM, int WN, int R, int C>
-constexpr uint32_t kernel_lds_bytes(int bits) {
-  const int e = 1 << bits;
-  const int lut = (32 * C * WN / (int)codes_per_group(bits) + 2) * e;
-  return (uint32_t)(2 * 32 * R * WM * 128 + lut * 2 + 4);
-}
-
 #define PK_F16_VARIANT(WM, WN, R, C)                                                              \
   F16Variant {                                                                                    \
     TileShape{WM, WN, R, C}, "pk_gemm_f16_b5_w" #WM "x" #WN "_m" #R "n" #C,                       \
         "pk_gemm_f16_b6_w" #WM "x" #WN "_m" #R "n" #C,                                            \
         {gemm_f16_kernel<5, WM, WN, R, C, false>, gemm_f16_kernel<6, WM, WN, R, C, false>},       \
-        {gemm_f16_kernel<5, WM, WN, R, C, true>, gemm_f16_kernel<6, WM, WN, R, C, true>},         \
-        kernel_lds_bytes<WM, WN, R, C>(6)                                                         \
+        {gemm_f16_kernel<5, WM, WN, R, C, true>, gemm_f16_kernel<6, WM, WN, R, C, true>}          \
   }
 
 const F16Variant kVariants[] = {
@@ -327,7 +319,6 @@ TileShape f16_variant(int index) { return variant_at(index).shape; }
 const char* f16_variant_name(int bits, int index) {
   return bits == 5 ? variant_at(index).name5 : variant_at(index).name6;
 }
-uint32_t f16_variant_lds_bytes(int index) { return variant_at(index).lds_bytes; }
 int f16_variant_family(int index) {
   if (index < kLocal) return kFamilyOperandOrder;
   return index < kLocal + f16k_variant_count() ? kFamilyPairCode : kFamilySmallM;
@@ -353,11 +344,9 @@ bool f16_group_streams(int index, uint32_t inner, uint32_t palette_groups, uint3
          f16s_group_streams(index - kLocal - f16k_variant_count(), inner, palette_groups, palette_group_columns);
 }
 
-uint32_t f16_group_launch_plan(int index, const SmallMGroupArgs& group, const char** kernel) {
-  void (*fn)(SmallMGroupArgs) = nullptr;
-  *kernel = nullptr;
+uint32_t f16_group_launch_plan(int index, const SmallMGroupArgs& group, GemmGroupKernel* kernel, const char** name) {
   if (f16_variant_family(index) != kFamilySmallM) return 0;
-  return f16s_group_launch(index - kLocal - f16k_variant_count(), group, &fn, kernel);
+  return f16s_group_launch(index - kLocal - f16k_variant_count(), group, kernel, name);
 }
 
 hipError_t launch_gemm_f16_group(int index, const SmallMGroupArgs& group, hipStream_t stream, hipEvent_t start,
@@ -371,16 +360,28 @@ bool f16_variant_streams(int bits, int variant, const GemmArgs& args) {
          f16::streams(variant_at(variant), bits, args);
 }
 
+GemmKernel f16_kernel(int bits, int variant, const GemmArgs& args, const char** name) {
+  const F16Variant& v = variant_at(variant);
+  *name = f16_variant_name(bits, variant);
+  switch (f16_variant_family(variant)) {
+    case kFamilySmallM: return f16s_kernel(bits, v, args, name);
+    case kFamilyPairCode: return f16k_kernel(bits, v, args);
+  }
+  return f16::single_path(v.shape, args) ? v.single[bits == 6] : v.general[bits == 6];
+}
+
+// A 1-D grid: row tiles x column tiles x K splits, or a small-M kernel's
+// work items padded to whole rounds of the eight XCDs.
 hipError_t launch_gemm_f16(int bits, int variant, const GemmArgs& args, hipStream_t stream, hipEvent_t start,
                            hipEvent_t stop) {
-  if (variant >= kLocal + f16k_variant_count())
-    return launch_gemm_f16s(bits, variant_at(variant), args, stream, start, stop);
-  if (variant >= kLocal) return launch_gemm_f16k(bits, variant_at(variant), args, stream, start, stop);
-  const F16Variant& v = variant_at(variant);
-  const uint32_t groups = tiles_m(v.shape, args.rows) * tiles_n(v.shape, args.columns) * args.splits;
+  const TileShape s = f16_variant(variant);
+  const uint32_t groups =
+      f16_variant_grid(variant, args.rows, args.columns, f16_variant_splits(variant) ? args.splits : 1u);
   if (groups == 0) return hipSuccess;
-  void (*kernel)(GemmArgs) = f16::single_path(v.shape, args) ? v.single[bits == 6] : v.general[bits == 6];
-  return launch_timed(kernel, dim3(groups), dim3(v.shape.threads()), stream, start, stop, args);
+  const char* name = nullptr;
+  const GemmKernel kernel = f16_kernel(bits, variant, args, &name);
+  if (!kernel) return hipErrorInvalidValue;
+  return launch_timed(kernel, dim3(groups), dim3(s.threads()), stream, start, stop, args);
 }
 
 }  // namespace pk

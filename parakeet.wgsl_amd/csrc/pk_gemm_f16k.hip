@@ -708,21 +708,12 @@ __global__ __launch_bounds__(256) void gemm_f16k_kernel(GemmArgs args) {
   }
 }
 
-template <int WN, int KS, int R, int C>
-constexpr uint32_t kernel_lds_bytes() {
-  constexpr int A_BYTES = 32 * R * kRowBytes;
-  constexpr int BLOCK_EX = KS * WN * C * 4 * 64 * 16;
-  constexpr int EX = pass_blocks(WN, KS, R, BLOCK_EX) * BLOCK_EX;
-  return (uint32_t)((EX > 3 * A_BYTES ? EX : 3 * A_BYTES) + kLutStride * 2 + 64 * 64 * 4);
-}
-
 #define PK_F16K_VARIANT(WN, KS, R, C, S, CLA, TAG)                                                              \
   F16Variant {                                                                                              \
     TileShape{1, WN, R, C, KS}, "pk_gemm_f16p_b5_n" #WN "k" #KS "_m" #R "n" #C TAG,                         \
         "pk_gemm_f16p_b6_n" #WN "k" #KS "_m" #R "n" #C TAG,                                                 \
         {gemm_f16k_kernel<5, WN, KS, R, C, false, S, CLA>, gemm_f16k_kernel<6, WN, KS, R, C, false, S, CLA>}, \
         {gemm_f16k_kernel<5, WN, KS, R, C, true, S, CLA>, gemm_f16k_kernel<6, WN, KS, R, C, true, S, CLA>},   \
-        kernel_lds_bytes<WN, KS, R, C>(),                                                                   \
         {gemm_f16k_kernel<5, WN, KS, R, C, false, S, CLA, true>,                                            \
          gemm_f16k_kernel<6, WN, KS, R, C, false, S, CLA, true>},                                           \
         {gemm_f16k_kernel<5, WN, KS, R, C, false, S, CLA, false, true>,                                     \
@@ -749,22 +740,13 @@ const F16Variant kVariants[] = {
 int f16k_variant_count() { return (int)(sizeof(kVariants) / sizeof(kVariants[0])); }
 const f16::F16Variant& f16k_variant(int index) { return kVariants[index]; }
 
-// Launch of a byte-code tile variant: a 1-D grid of row tiles x column
-// tiles; the `single` kernel needs K % 64 == 0 and every tile inside one
-// palette group.
-hipError_t launch_gemm_f16k(int bits, const f16::F16Variant& v, const GemmArgs& args, hipStream_t stream,
-                            hipEvent_t start, hipEvent_t stop) {
-  const uint32_t groups = tiles_m(v.shape, args.rows) * tiles_n(v.shape, args.columns);
-  if (groups == 0) return hipSuccess;
+// The `single` kernel needs K % 64 == 0 and every tile inside one palette
+// group; the fused row norm that path and K staged in LDS.
+GemmKernel f16k_kernel(int bits, const f16::F16Variant& v, const GemmArgs& args) {
   const bool single = f16::single_path(v.shape, args);
-  if (args.norm_columns) {
-    // The fused row norm needs the fixed-palette path and K staged in LDS.
-    if (!single || args.inner > kNormMaxInner || !v.normed[bits == 6]) return hipErrorInvalidValue;
-    return launch_timed(v.normed[bits == 6], dim3(groups), dim3(v.shape.threads()), stream, start, stop, args);
-  }
-  void (*kernel)(GemmArgs) = single ? v.single[bits == 6] : v.general[bits == 6];
-  if (f16::streams(v, bits, args)) kernel = v.streamed[bits == 6];
-  return launch_timed(kernel, dim3(groups), dim3(v.shape.threads()), stream, start, stop, args);
+  if (args.norm_columns) return single && args.inner <= kNormMaxInner ? v.normed[bits == 6] : nullptr;
+  if (f16::streams(v, bits, args)) return v.streamed[bits == 6];
+  return single ? v.single[bits == 6] : v.general[bits == 6];
 }
 
 }  // namespace pk

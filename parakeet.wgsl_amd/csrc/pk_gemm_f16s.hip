@@ -757,8 +757,7 @@ struct SmallMVariant {
     TileShape{1, 1, RW, CB, W}, "pk_gemm_f16s_b5_k" #W "_m" #RW "n" #CB "d" #D,                           \
         "pk_gemm_f16s_b6_k" #W "_m" #RW "n" #CB "d" #D,                                                    \
         {gemm_f16s_kernel<5, W, RW, CB, D, false, false>, gemm_f16s_kernel<6, W, RW, CB, D, false, false>}, \
-        {gemm_f16s_kernel<5, W, RW, CB, D, true, false>, gemm_f16s_kernel<6, W, RW, CB, D, true, false>},   \
-        (uint32_t)sizeof(SmallMShared<W, RW, CB>)                                                          \
+        {gemm_f16s_kernel<5, W, RW, CB, D, true, false>, gemm_f16s_kernel<6, W, RW, CB, D, true, false>}    \
   }
 #define PK_F16S_VARIANT(W, RW, CB, D)                                                                      \
   SmallMVariant {                                                                                          \
@@ -819,16 +818,10 @@ int f16s_variant_count() { return (int)(sizeof(kVariants) / sizeof(kVariants[0])
 const f16::F16Variant& f16s_variant(int index) { return kVariants[index].v; }
 const char* f16s_group_name(int index) { return kVariants[index].group_name; }
 
-// One workgroup per (column group, row group), padded to whole rounds of the
-// eight XCDs. The `single` kernel needs K % 64 == 0 and the CB * 32
-// columns of an item inside one palette group.
-hipError_t launch_gemm_f16s(int bits, const f16::F16Variant& v, const GemmArgs& args, hipStream_t stream,
-                            hipEvent_t start, hipEvent_t stop) {
-  const uint32_t cgs = tiles_n(v.shape, args.columns);
-  if (cgs == 0 || args.rows == 0) return hipSuccess;
-  const bool single = (args.inner & 63u) == 0u &&
-                      (args.palette_groups == 1 || args.palette_group_columns % (uint32_t)v.shape.tile_columns() == 0);
-  void (*kernel)(GemmArgs) = single ? v.single[bits == 6] : v.general[bits == 6];
+// The `single` kernel needs K % 64 == 0 and the CB * 32 columns of an item
+// inside one palette group.
+GemmKernel f16s_kernel(int bits, const f16::F16Variant& v, const GemmArgs& args, const char** name) {
+  const bool single = f16::single_path(v.shape, args);
   // More than one row group of the 32 x 32 tile and K from 768 on: the rows
   // come through LDS (same sums). 188 x 4096 -> 1024 12.1 -> 9.6 us, 64 x 4096
   // -> 1024 11.3 -> 8.8, 188 x 1024 -> 1024 6.1 -> 5.5, 64 x 896 -> 1024 5.5 ->
@@ -836,10 +829,12 @@ hipError_t launch_gemm_f16s(int bits, const f16::F16Variant& v, const GemmArgs& 
   // its four rows of loads ahead in vain (188 x 512 -> 512 3.9 -> 4.7, 64 x 640
   // -> 1024 4.6 -> 4.9), and with one row group (16 rows) the turn costs more
   // than it saves, 5.0 against 5.2 us for 1024 -> 4096.
-  if (single && args.rows > 32u && args.inner >= 768u && v.shape.m_blocks == 1 && v.shape.n_blocks == 1 && v.shape.k_split == 8)
-    kernel = bits == 6 ? gemm_f16s_kernel<6, 8, 1, 1, 4, false, true> : gemm_f16s_kernel<5, 8, 1, 1, 4, false, true>;
-  return launch_timed(kernel,
-                      dim3(small_m_grid(v.shape, cgs, args.rows)), dim3(v.shape.threads()), stream, start, stop, args);
+  if (single && args.rows > 32u && args.inner >= 768u && v.shape.m_blocks == 1 && v.shape.n_blocks == 1 &&
+      v.shape.k_split == 8) {
+    *name = bits == 6 ? "pk_gemm_f16s_b6_k8_m1n1d4rows" : "pk_gemm_f16s_b5_k8_m1n1d4rows";
+    return bits == 6 ? gemm_f16s_kernel<6, 8, 1, 1, 4, false, true> : gemm_f16s_kernel<5, 8, 1, 1, 4, false, true>;
+  }
+  return single ? v.single[bits == 6] : v.general[bits == 6];
 }
 
 bool f16s_group_persistent(int index) { return kVariants[index].stream != nullptr; }
@@ -854,7 +849,7 @@ bool f16s_group_streams(int index, uint32_t inner, uint32_t palette_groups, uint
 // The kernel and grid a group launch runs: the persistent kernel on at most
 // one round of resident workgroups when the variant has one and the host
 // set g.persistent (every member eligible), else one workgroup per item.
-uint32_t f16s_group_launch(int index, const SmallMGroupArgs& g, void (**kernel)(SmallMGroupArgs), const char** name) {
+uint32_t f16s_group_launch(int index, const SmallMGroupArgs& g, GemmGroupKernel* kernel, const char** name) {
   const SmallMVariant& sv = kVariants[index];
   const uint32_t items = small_m_grid(sv.v.shape, g.items_count, g.rows);
   if (sv.stream && g.persistent) {
@@ -873,7 +868,7 @@ uint32_t f16s_group_launch(int index, const SmallMGroupArgs& g, void (**kernel)(
 hipError_t launch_gemm_f16s_group(int index, const SmallMGroupArgs& g, hipStream_t stream, hipEvent_t start,
                                   hipEvent_t stop) {
   if (g.items_count == 0 || g.rows == 0) return hipSuccess;
-  void (*kernel)(SmallMGroupArgs) = nullptr;
+  GemmGroupKernel kernel = nullptr;
   const char* name = nullptr;
   const dim3 grid(f16s_group_launch(index, g, &kernel, &name)), block(kVariants[index].v.shape.threads());
   if (start || stop)

@@ -516,6 +516,10 @@ const char* f32_variant_name(int bits, int index) {
   return bits == 5 ? kVariants[index].name5 : kVariants[index].name6;
 }
 
+GemmKernel f32_kernel(int bits, int variant) {
+  return bits == 5 ? kVariants[variant].kernel5 : kVariants[variant].kernel6;
+}
+
 hipError_t launch_gemm_f32(int bits, int variant, const GemmArgs& args, hipStream_t stream, hipEvent_t start,
                            hipEvent_t stop) {
   const Variant& v = kVariants[variant];
@@ -523,7 +527,7 @@ hipError_t launch_gemm_f32(int bits, int variant, const GemmArgs& args, hipStrea
   const dim3 grid((n_pad + v.shape.tile_columns() - 1) / v.shape.tile_columns(),
                   (args.rows + v.shape.tile_rows() - 1) / v.shape.tile_rows());
   if (grid.y == 0) return hipSuccess;
-  return launch_timed(bits == 5 ? v.kernel5 : v.kernel6, grid, dim3(v.shape.threads()), stream, start, stop, args);
+  return launch_timed(f32_kernel(bits, variant), grid, dim3(v.shape.threads()), stream, start, stop, args);
 }
 
 }  // namespace pk

@@ -204,7 +204,9 @@ hipError_t launch_relayout(int bits, const uint32_t* src, int src_parts, uint32_
 int f16_variant_count();
 TileShape f16_variant(int index);
 const char* f16_variant_name(int bits, int index);
-uint32_t f16_variant_lds_bytes(int index);
+// The kernel launch_gemm_f16 runs for `args` and its name (null: refused).
+typedef void (*GemmKernel)(GemmArgs);
+GemmKernel f16_kernel(int bits, int variant, const GemmArgs& args, const char** name);
 // Kernel family of an f16 variant. Only the operand-order family also runs
 // split-K across workgroups; the others split K inside the workgroup.
 enum F16Family : int { kFamilyOperandOrder = 0, kFamilyPairCode = 1, kFamilySmallM = 2 };
@@ -248,14 +250,16 @@ bool f16_group_persistent(int index);
 // persistent group kernel of small-M variant `index` (false for a variant
 // without one).
 bool f16_group_streams(int index, uint32_t inner, uint32_t palette_groups, uint32_t palette_group_columns);
-// Grid (x) and kernel name of the launch launch_gemm_f16_group makes.
-uint32_t f16_group_launch_plan(int index, const SmallMGroupArgs& group, const char** kernel);
+// Grid (x), kernel and its name of the launch launch_gemm_f16_group makes.
+typedef void (*GemmGroupKernel)(SmallMGroupArgs);
+uint32_t f16_group_launch_plan(int index, const SmallMGroupArgs& group, GemmGroupKernel* kernel, const char** name);
 hipError_t launch_gemm_f16_group(int index, const SmallMGroupArgs& group, hipStream_t stream,
                                  hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
 
 int f32_variant_count();
 TileShape f32_variant(int index);
 const char* f32_variant_name(int bits, int index);
+GemmKernel f32_kernel(int bits, int variant);
 hipError_t launch_gemm_f32(int bits, int variant, const GemmArgs& args, hipStream_t stream,
                            hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
 
