@@ -67,10 +67,13 @@ __device__ __forceinline__ half8 load_position(const _Float16* positions, uint32
 
 __device__ __forceinline__ float fast_exp(float x) { return __builtin_amdgcn_exp2f(x * 1.4426950408889634f); }
 
+// Windows of at most so many frames load each key tile when it is used.
+constexpr uint32_t kLoadAheadFrames = 256;
+
 // Headroom of the lazily moved softmax maximum (natural-log units).
 constexpr float kRescaleMargin = 8.0f;
 
-template <int KSPLIT, bool ROW_MAJOR>
+template <int KSPLIT, bool ROW_MAJOR, bool AHEAD>
 __global__ __launch_bounds__(64 * KSPLIT) void rel_attention_f16_kernel(AttnArgs args) {
   __shared__ __attribute__((aligned(16))) uint8_t smem[KSPLIT * kWaveLds];
   const int lane = threadIdx.x & 63;
@@ -97,16 +100,17 @@ __global__ __launch_bounds__(64 * KSPLIT) void rel_attention_f16_kernel(AttnArgs
     return;
   }
 
-  // A key tile's rows, all loads before any use, the next tile's as soon as
-  // the products have read this one's (clamped, unconditional): with one
-  // wavefront per SIMD only these loads overlap the softmax and the PV
-  // products. 256 VGPRs + 230 AGPRs; 1 x 188 12.2 -> 11.8 us, 5 x 188 14.9 ->
-  // 13.5, 1 x 750 33.9 -> 26.7 (1 x 100, one tile per wavefront, 9.1 -> 9.3). The
-  // first tile's loads ahead of the query operands as well: 12.1, 1 x 60 9.3
-  // against 7.6.
+  // A key tile's rows, all loads of a kind before any use. AHEAD (long
+  // windows): the next tile's as soon as the products have read this one's,
+  // unconditional, so that with one wavefront per SIMD these loads overlap the
+  // softmax and the PV products (256 VGPRs + 230 AGPRs): 1 x 400 20.7 -> 17.6 us
+  // against loading each tile when it is used, 2 x 400 20.7 -> 18.7, 3 x 260
+  // 17.6 -> 16.8, 1 x 750 20.9 -> 20.1, the same at 1 x 300. Up to 256 frames a wavefront has two tiles at most and
+  // their values ahead of the products only delay those: 1 x 188 10.1 -> 9.95,
+  // 1 x 60 7.85 -> 7.4, 5 x 188 12.0 -> 11.75 without.
   const int tiles = (live + kTile - 1) / kTile;
   half8 kv[8], ra[8], rb[8], vx[8];
-  auto load_tile = [&](int kt) {
+  auto load_keys = [&](int kt) {
     const int k0 = kt * kTile;
     const int p_lo = T - 1 - q0 - (kTile - 1) + k0;
     const int pmax = (int)args.position_rows - 1;
@@ -119,8 +123,11 @@ __global__ __launch_bounds__(64 * KSPLIT) void rel_attention_f16_kernel(AttnArgs
       ra[s] = load_position<ROW_MAJOR>(static_cast<const _Float16*>(args.positions), args.position_rows, head, pa, d0);
       rb[s] = load_position<ROW_MAJOR>(static_cast<const _Float16*>(args.positions), args.position_rows, head, pb, d0);
     }
+  };
+  auto load_values = [&](int kt) {
+    const _Float16* vrow = qkv + (uint64_t)min(kt * kTile + j, T - 1) * kQkvRow + 2 * kHidden;
 #pragma unroll
-    for (int c = 0; c < 8; ++c) vx[c] = load8(krow + kHidden + 16 * c + 8 * hh);
+    for (int c = 0; c < 8; ++c) vx[c] = load8(vrow + 16 * c + 8 * hh);
   };
 
   // (Q+u)^T and (Q+v)^T operands of query q0 + j: channels 16s + 8hh + 0..7.
@@ -159,13 +166,17 @@ __global__ __launch_bounds__(64 * KSPLIT) void rel_attention_f16_kernel(AttnArgs
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[db][r] = 0.0f;
 
-  load_tile(min(wave, tiles - 1));
+  if (AHEAD && wave < tiles) {
+    load_keys(wave);
+    load_values(wave);
+  }
   for (int kt = wave; kt < tiles; kt += KSPLIT) {
     const int k0 = kt * kTile;
     // S^T = K (Q+u)^T and W^T = R[p_lo ..] (Q+v)^T.
     floatx16 ac, w0, w1;
 #pragma unroll
     for (int r = 0; r < 16; ++r) ac[r] = w0[r] = w1[r] = 0.0f;
+    if constexpr (!AHEAD) load_keys(kt);
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
       ac = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv[s], qu[s], ac, 0, 0, 0);
@@ -173,6 +184,7 @@ __global__ __launch_bounds__(64 * KSPLIT) void rel_attention_f16_kernel(AttnArgs
       w1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(rb[s], qv[s], w1, 0, 0, 0);
     }
     // V tile -> LDS, transposed: vt[d][swap23(key)].
+    if constexpr (!AHEAD) load_values(kt);
     {
       const int slot = (j & ~12) | ((j & 4) << 1) | ((j & 8) >> 1);
 #pragma unroll
@@ -182,7 +194,10 @@ __global__ __launch_bounds__(64 * KSPLIT) void rel_attention_f16_kernel(AttnArgs
         for (int t = 0; t < 8; ++t) vt[(d0 + t) * kVtStride + slot] = vx[c][t];
       }
     }
-    if (kt + KSPLIT < tiles) load_tile(kt + KSPLIT);
+    if (AHEAD && kt + KSPLIT < tiles) {
+      load_keys(kt + KSPLIT);
+      load_values(kt + KSPLIT);
+    }
     // Window rows c = 32 blk + 8 (r/4) + 4 hh + r%4, column j.
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
@@ -865,8 +880,8 @@ struct AttnVariant {
 
 #define PK_ATTN_VARIANT(K)                                                                                 \
   AttnVariant {                                                                                            \
-    "pk_rel_attention_f16_q32_w" #K, K, kTile, (uint32_t)(K * kWaveLds), rel_attention_f16_kernel<K, false>, \
-        rel_attention_f16_kernel<K, true>                                                                  \
+    "pk_rel_attention_f16_q32_w" #K, K, kTile, (uint32_t)(K * kWaveLds),                                    \
+        rel_attention_f16_kernel<K, false, true>, rel_attention_f16_kernel<K, true, true>                  \
   }
 #define PK_ATTN_SHARED_VARIANT(NQ)                                                                         \
   AttnVariant {                                                                                            \
@@ -947,6 +962,9 @@ hipError_t launch_attention(bool f16, int variant, const AttnArgs& base, uint32_
   args.work_items = batch * kHeads * g.query_tiles;
   const AttnVariant& v = f16 ? kF16Variants[variant] : kF32Variants[variant];
   void (*kernel)(AttnArgs) = base.positions_row_major ? v.row_major : v.packed;
+  if (f16 && variant == 0 && base.frames <= kLoadAheadFrames)
+    kernel = base.positions_row_major ? rel_attention_f16_kernel<4, true, false>
+                                      : rel_attention_f16_kernel<4, false, false>;
   if (start || stop)
     hipExtLaunchKernelGGL(kernel, dim3(g.grid), dim3(g.block_threads), 0, stream, start, stop, 0, args);
   else

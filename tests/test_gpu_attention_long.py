@@ -1,6 +1,6 @@
-"""Windows longer than 256 frames in every planned range of query tiles (few:
-key-split wavefronts with the next tile prefetched, then the shared kernels),
-at tile edges, against the oracle."""
+"""Windows around and above 256 frames in every planned range of query tiles
+(few: key-split wavefronts, above 256 frames with the next tile prefetched,
+then the shared kernels), at tile edges, against the oracle."""
 import pytest
 
 from test_gpu_attention import assert_attention_parity, run_attention
@@ -18,6 +18,7 @@ def scope(ctx):
 
 @pytest.mark.parametrize("row_major", [False, True])
 @pytest.mark.parametrize("batch,frames,valid,kernel", [
+    (1, 33, [33], "q32_w4"), (2, 129, [129, 1], "q32_w4"), (3, 256, [256, 0, 65], "q32_w4"),
     (1, 257, [257], "q32_w4"), (2, 300, [289, 33], "q32_w4"), (1, 1024, [1000], "q32_w4"),
     (4, 320, [320, 1, 129, 0], "q2x32_shared"), (5, 320, [320, 64, 200, 31, 96], "q4x32_shared")])
 def test_long_windows_match_oracle(abi, ctx, scope, oracle, workloads, batch, frames, valid, kernel, row_major):
