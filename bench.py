@@ -1032,6 +1032,7 @@ def run_encoder(args, abi, ctx, decoder=False):
                    **abi.decode_tdt_status(meta[stack.batch:stack.batch + active]),
                    "kernel": "tdt_resident_kernel" if tdt.resident_windows() else
                              "tdt_team_kernel" if tdt.team_size() > 1 else "tdt_decode_kernel",
+                   "abandoned_launches": tdt.abandoned_launches(),
                    "max_tokens": 1024}
     dense = None
     if not args.no_dense and not f32:

@@ -137,10 +137,16 @@ int pk_tdt_enqueue_timed(pk_tdt_op *op, uint32_t active_batch, void *stream, voi
 int pk_tdt_set_team_size(pk_tdt_op *op, uint32_t members);
 int pk_tdt_team_size(const pk_tdt_op *op, uint32_t *members);
 /* Windows of one resident launch of this op, 0 if it does not decode that
-   way; and the polls one of its waits makes before the launch is given up
-   (for tests: 0 gives up at the first unsuccessful poll). */
+   way; and how many launches of its latest decode were given up (read once
+   that decode has completed). */
 int pk_tdt_resident_windows(const pk_tdt_op *op, uint32_t *windows);
+int pk_tdt_abandoned_launches(const pk_tdt_op *op, uint32_t *launches);
+/* For tests: the polls a wait of a resident launch makes before the launch is
+   given up (0: the first unsuccessful one), and the 100 MHz ticks its
+   workgroups wait for each other at the start (0: not at all, the launch is
+   given up). */
 int pk_tdt_set_wait_limit(pk_tdt_op *op, uint32_t polls);
+int pk_tdt_set_join_limit(pk_tdt_op *op, uint32_t ticks);
 /* Idempotent; frees the team buffers (after the device has drained), and
    enqueue after destroy returns PK_DESTROYED. Enqueue on a stream that is
    capturing a graph returns PK_INVALID_ARGUMENT. */

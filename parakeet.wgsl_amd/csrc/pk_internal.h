@@ -438,7 +438,7 @@ struct TdtResident {
   uint64_t* exchange;    // [batch, kTdtResidentWords], right after the sync words; cleared per decode
   uint32_t base, windows;  // of one launch
   uint32_t spin_limit;   // polls before a wait gives up
-  uint64_t join_ticks;   // 100 MHz ticks before the members stop waiting for each other at the start
+  uint64_t join_ticks;   // 100 MHz ticks before the members stop waiting for each other at the start (0: at once)
 };
 uint32_t tdt_resident_windows(bool f32);
 bool tdt_resident_fits(int device, bool f32);

@@ -21,6 +21,7 @@ struct pk_tdt_op {
   pk::TdtTeam team{};   // members == 0: one workgroup per window
   uint32_t* team_memory = nullptr;
   pk::TdtResident resident{};  // sync null: the team's or the window's own workgroups decode
+  bool resident_decoded = false;  // a resident decode was enqueued: its abort words mean something
   bool destroyed = false;
 };
 
@@ -114,6 +115,7 @@ void free_team(pk_tdt_op* op) {
   op->team_memory = nullptr;
   op->team = pk::TdtTeam{};
   op->resident = pk::TdtResident{};
+  op->resident_decoded = false;
 }
 
 // Gives an op whose team size was left to the library (0) the resident
@@ -317,6 +319,25 @@ int pk_tdt_set_wait_limit(pk_tdt_op* op, uint32_t polls) {
   return ok();
 }
 
+int pk_tdt_set_join_limit(pk_tdt_op* op, uint32_t ticks) {
+  if (!op) return fail(PK_INVALID_ARGUMENT, "TDT decoder op is null");
+  if (op->destroyed) return fail(PK_DESTROYED, "%s was destroyed", op->label.c_str());
+  op->resident.join_ticks = ticks;
+  return ok();
+}
+
+int pk_tdt_abandoned_launches(const pk_tdt_op* op, uint32_t* launches) {
+  if (!op || !launches) return fail(PK_INVALID_ARGUMENT, "TDT decoder op or output is null");
+  *launches = 0;
+  if (!op->resident_decoded) return ok();
+  uint32_t words[2 * pk::kTdtResidentLaunches * pk::kTdtSyncStride];
+  PK_HIP(hipSetDevice(op->ctx->device), "hipSetDevice");
+  PK_HIP(hipMemcpy(words, op->resident.sync, sizeof words, hipMemcpyDeviceToHost), "hipMemcpy");
+  for (uint32_t i = 0; i < pk::kTdtResidentLaunches; ++i)
+    *launches += words[(2 * i + 1) * pk::kTdtSyncStride] != 0u;
+  return ok();
+}
+
 int pk_tdt_enqueue(pk_tdt_op* op, uint32_t active_batch, void* stream) {
   return pk_tdt_enqueue_timed(op, active_batch, stream, nullptr, nullptr);
 }
@@ -339,6 +360,7 @@ int pk_tdt_enqueue_timed(pk_tdt_op* op, uint32_t active_batch, void* stream, voi
   if (op->resident.sync) {
     PK_HIP(launch_in_turn(op, batch, s, static_cast<hipEvent_t>(start_event), static_cast<hipEvent_t>(end_event)),
            "resident TDT decoder launch");
+    op->resident_decoded = true;
     return ok();
   }
   if (op->team.members) {

@@ -836,9 +836,9 @@ __global__ __launch_bounds__(kBlock) void tdt_resident_kernel(TdtArgs a, TdtResi
   if (threadIdx.x == 0) {
     const uint64_t start = wall_clock64();
     uint32_t failed = 0;
-    while (xload(joined) < G::kMembers) {
+    while (r.join_ticks == 0 || xload(joined) < G::kMembers) {
       failed = xload(abort);
-      if (!failed && wall_clock64() - start > r.join_ticks) {
+      if (!failed && wall_clock64() - start >= r.join_ticks) {
         xstore(abort, 1u);
         failed = 1;
       }

@@ -549,7 +549,9 @@ SIGNATURES = {
     "pk_tdt_release": (ctypes.c_int, [_VP]),
     "pk_tdt_set_team_size": (ctypes.c_int, [_VP, ctypes.c_uint32]),
     "pk_tdt_resident_windows": (ctypes.c_int, [_VP, ctypes.POINTER(ctypes.c_uint32)]),
+    "pk_tdt_abandoned_launches": (ctypes.c_int, [_VP, ctypes.POINTER(ctypes.c_uint32)]),
     "pk_tdt_set_wait_limit": (ctypes.c_int, [_VP, ctypes.c_uint32]),
+    "pk_tdt_set_join_limit": (ctypes.c_int, [_VP, ctypes.c_uint32]),
     "pk_graph_begin_capture": (ctypes.c_int, [_VP, _VP]),
     "pk_graph_end_capture": (ctypes.c_int, [_VP, _VP, _PPV]),
     "pk_graph_launch": (ctypes.c_int, [_VP, _VP]),
@@ -1271,9 +1273,19 @@ class TdtDecoderOp:
         check(load().pk_tdt_resident_windows(self.handle, ctypes.byref(out)))
         return out.value
 
+    def abandoned_launches(self) -> int:
+        """Resident launches of the latest decode that were given up (once it has completed)."""
+        out = ctypes.c_uint32()
+        check(load().pk_tdt_abandoned_launches(self.handle, ctypes.byref(out)))
+        return out.value
+
     def set_wait_limit(self, polls: int) -> None:
         """Polls before a resident launch is given up (and decoded by one workgroup per window)."""
         check(load().pk_tdt_set_wait_limit(self.handle, polls))
+
+    def set_join_limit(self, ticks: int) -> None:
+        """100 MHz ticks a resident launch waits for its workgroups at the start (0: given up)."""
+        check(load().pk_tdt_set_join_limit(self.handle, ticks))
 
     def destroy(self) -> None:
         check(load().pk_tdt_destroy(self.handle))

@@ -39,7 +39,7 @@ class Decoder:
         return {n: b.download().view(np.uint32) for n, b in self.out.items()}
 
 
-def decode(abi, scope, ctx, case, precision, *, team=None, polls=None, active=0):
+def decode(abi, scope, ctx, case, precision, *, team=None, polls=None, join=None, active=0):
     d = Decoder(abi, scope, ctx, case, precision)
     try:
         if team is not None:
@@ -47,9 +47,15 @@ def decode(abi, scope, ctx, case, precision, *, team=None, polls=None, active=0)
         assert bool(d.op.resident_windows()) == (team is None)
         if polls is not None:
             d.op.set_wait_limit(polls)
-        print(precision, "batch", case.batch, "team", team, "polls", polls, flush=True)
+        if join is not None:
+            d.op.set_join_limit(join)
+        print(precision, "batch", case.batch, "team", team, "polls", polls, "join", join, flush=True)
+        assert d.op.abandoned_launches() == 0
         d.op.enqueue(active)
         ctx.synchronize()
+        given_up = polls is not None or join is not None
+        launches = -(-(active or case.batch) // d.op.resident_windows()) if given_up else 0
+        assert d.op.abandoned_launches() == launches
         return d.words()
     finally:
         d.op.release()
@@ -90,10 +96,11 @@ def test_resident_decode_leaves_out_zero_inputs_of_weights_that_are_not_finite(a
     same(decode(abi, scope, ctx, case, precision), decode(abi, scope, ctx, case, precision, team=1))
 
 
+@pytest.mark.parametrize("limit", ["polls", "join"])
 @pytest.mark.parametrize("precision,batch", [("f16", 3), ("f16", 33), ("f32", 7)])
-def test_resident_decode_that_gives_up_is_decoded_again(abi, ctx, scope, workloads, precision, batch):
+def test_resident_decode_that_gives_up_is_decoded_again(abi, ctx, scope, workloads, precision, batch, limit):
     case = ragged(workloads, 40 + batch, batch, precision, 0.5)
-    same(decode(abi, scope, ctx, case, precision, polls=0), decode(abi, scope, ctx, case, precision, team=1))
+    same(decode(abi, scope, ctx, case, precision, **{limit: 0}), decode(abi, scope, ctx, case, precision, team=1))
 
 
 def test_resident_decodes_on_two_streams_and_an_active_prefix(abi, ctx, scope, workloads):
@@ -112,6 +119,7 @@ def test_resident_decodes_on_two_streams_and_an_active_prefix(abi, ctx, scope, w
         ctx.synchronize()
         ctx.synchronize(other)
         for d, w in zip(ops, want):
+            assert d.op.abandoned_launches() == 0
             same(d.words(), w)
     finally:
         for d in ops:
