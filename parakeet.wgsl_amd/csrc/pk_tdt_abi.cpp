@@ -127,7 +127,6 @@ int set_resident(pk_tdt_op* op) {
   if (op->batch > windows || op->ctx->device < 0 || op->ctx->device >= kMaxDevices || !pk::tdt_resident_fits(op->ctx->device, op->f32)) return PK_OK;
   const uint64_t sync_words = 2ull * pk::kTdtResidentLaunches * pk::kTdtSyncStride;
   uint32_t* memory = nullptr;
-  PK_HIP(hipSetDevice(op->ctx->device), "hipSetDevice");
   if (hipMalloc(reinterpret_cast<void**>(&memory), sync_words * 4 + (uint64_t)op->batch * pk::kTdtResidentWords * 8) !=
       hipSuccess) {
     (void)hipGetLastError();
@@ -145,7 +144,6 @@ int set_team(pk_tdt_op* op, uint32_t members) {
   if (members == 0) return PK_OK;
   const uint64_t sync_words = 2ull * op->batch * pk::kTdtSyncStride;
   const uint64_t words = sync_words + (uint64_t)op->batch * 2 * members * 4;
-  PK_HIP(hipSetDevice(op->ctx->device), "hipSetDevice");
   const hipError_t e = hipMalloc(reinterpret_cast<void**>(&op->team_memory), words * 4);
   if (e != hipSuccess)
     return fail(PK_ALLOCATION_FAILURE, "%s: cannot allocate the decoder's team buffers: %s", op->label.c_str(),
@@ -264,6 +262,7 @@ int pk_tdt_create(pk_context* ctx, const pk_tdt_desc* d, pk_tdt_op** out) {
   if (!out) return fail(PK_INVALID_ARGUMENT, "output pointer is null");
   *out = nullptr;
   if (int s = validate(d)) return s;
+  PK_HIP(hipSetDevice(ctx->device), "hipSetDevice");  // the occupancy queries below ask the current device
   auto* op = new pk_tdt_op();
   op->ctx = ctx;
   op->label = d->label ? d->label : "parakeet-persistent-tdt-decode";
@@ -284,6 +283,7 @@ int pk_tdt_create(pk_context* ctx, const pk_tdt_desc* d, pk_tdt_op** out) {
 int pk_tdt_set_team_size(pk_tdt_op* op, uint32_t members) {
   if (!op) return fail(PK_INVALID_ARGUMENT, "TDT decoder op is null");
   if (op->destroyed) return fail(PK_DESTROYED, "%s was destroyed", op->label.c_str());
+  PK_HIP(hipSetDevice(op->ctx->device), "hipSetDevice");
   const bool chosen = members == 0;
   if (chosen) members = choose_members(op->ctx->device, op->batch, op->f32);
   else if (members == 1) members = 0;
@@ -295,7 +295,6 @@ int pk_tdt_set_team_size(pk_tdt_op* op, uint32_t members) {
   else if ((uint64_t)op->batch * members > pk::tdt_team_capacity(op->ctx->device))
     return fail(PK_RANGE_ERROR, "%s: %u windows x %u workgroups cannot be resident together", op->label.c_str(),
                 op->batch, members);
-  PK_HIP(hipSetDevice(op->ctx->device), "hipSetDevice");
   if (int s = set_team(op, members)) return s;
   return chosen ? set_resident(op) : PK_OK;
 }
@@ -401,6 +400,7 @@ int pk_tdt_decode_static(pk_context* ctx, const pk_tdt_desc* d, uint32_t members
   if (batch > kStaticWindows)
     return fail(PK_RANGE_ERROR, "%s: %u windows exceed the %u of the static decoder buffers", label, batch,
                 kStaticWindows);
+  PK_HIP(hipSetDevice(ctx->device), "hipSetDevice");
   const bool f32 = d->precision == PK_PRECISION_F32;
   if (members == 0) members = choose_members(ctx->device, batch, f32);
   else if (members == 1) members = 0;
@@ -410,7 +410,6 @@ int pk_tdt_decode_static(pk_context* ctx, const pk_tdt_desc* d, uint32_t members
     return fail(PK_RANGE_ERROR, "%s: team decoding is built for the f16 profile (f32 team size 1)", label);
   else if ((uint64_t)batch * members > pk::tdt_team_capacity(ctx->device))
     return fail(PK_RANGE_ERROR, "%s: %u windows x %u workgroups cannot be resident together", label, batch, members);
-  PK_HIP(hipSetDevice(ctx->device), "hipSetDevice");
   const hipStream_t st = stream_or_default(ctx, stream);
   const pk::TdtArgs args = args_of(d);
   if (members == 0) {
