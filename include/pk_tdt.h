@@ -119,11 +119,13 @@ int pk_tdt_enqueue_timed(pk_tdt_op *op, uint32_t active_batch, void *stream, voi
    workgroup on each of 160 (f16) or 214 (f32) compute units and decodes up to
    16 (f16) or 6 (f32) windows per launch with them, up to four launches. Its
    workgroups wait for each other, never without a bound: they give up after
-   10 ms at the start (another kernel holds their compute units) or after
-   2^20 polls later, and a kernel behind them in the stream then decodes the
-   windows with one workgroup each, so such a decode is late but complete and
-   never ends with PK_TDT_SYNC_TIMEOUT. Resident decodes of one process on one
-   GPU run one after the other (an event wait on the stream).
+   10 ms (f32: 20 ms) at the start, when another kernel holds their compute
+   units, or after 2^20 polls later. Kernels behind them in the stream then
+   decode the windows, in f16 a team of pk_tdt_team_size workgroups each, and
+   where that gives up too (2^16 polls), and in f32, one workgroup each. Such
+   a decode is late but complete and never ends with PK_TDT_SYNC_TIMEOUT.
+   Resident decodes of one process on one GPU run one after the other (an
+   event wait on the stream).
    A team launch is an ordinary launch whose grid fits the workgroups an
    idle device holds at once: kernels running on other streams at the same
    time can keep members from being resident, and a barrier that then
@@ -144,9 +146,10 @@ int pk_tdt_abandoned_launches(const pk_tdt_op *op, uint32_t *launches);
 /* For tests: the polls a wait of a resident launch makes before the launch is
    given up (0: the first unsuccessful one), and the 100 MHz ticks its
    workgroups wait for each other at the start (0: not at all, the launch is
-   given up). */
+   given up); and the polls of a barrier of the teams behind it. */
 int pk_tdt_set_wait_limit(pk_tdt_op *op, uint32_t polls);
 int pk_tdt_set_join_limit(pk_tdt_op *op, uint32_t ticks);
+int pk_tdt_set_team_limit(pk_tdt_op *op, uint32_t polls);
 /* Idempotent; frees the team buffers (after the device has drained), and
    enqueue after destroy returns PK_DESTROYED. Enqueue on a stream that is
    capturing a graph returns PK_INVALID_ARGUMENT. */

@@ -392,10 +392,12 @@ struct TdtArgs {
   uint32_t *tokens, *token_frames, *token_durations;  // [batch, max_tokens]
   uint32_t *counts, *status;     // [batch]
   uint32_t frames, max_tokens;
-  // tdt_decode_kernel behind resident launches: window b is decoded only if
-  // word 2 * (b / aborted_windows) * kTdtSyncStride is not 0 (null: always).
+  // The kernels behind resident launches decode window b only if word
+  // 2 * (b / aborted_windows) * kTdtSyncStride is not 0 (null: always), and
+  // tdt_decode_kernel behind the teams only if its team gave up as well.
   const uint32_t* aborted;
   uint32_t aborted_windows;
+  uint32_t after_team;
 };
 // One workgroup per window; `f32` selects the f32 profile's kernel.
 hipError_t launch_tdt_decode(const TdtArgs& args, uint32_t batch, bool f32, hipStream_t stream,
@@ -417,8 +419,9 @@ struct TdtTeam {
 bool tdt_team_members_supported(uint32_t members);
 // Team workgroups that can be resident at once on `device` (0 if unknown).
 uint32_t tdt_team_capacity(int device);
+// `cleared`: team.sync is zero already.
 hipError_t launch_tdt_team(const TdtArgs& args, const TdtTeam& team, uint32_t batch, hipStream_t stream,
-                           hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
+                           hipEvent_t start = nullptr, hipEvent_t stop = nullptr, bool cleared = false);
 
 // Resident decoding (pk_tdt_resident.hip, both profiles): the weights held in
 // the LDS of one workgroup per compute unit, all windows of a launch sharing
@@ -435,7 +438,9 @@ constexpr uint32_t kTdtResidentH0 = 0, kTdtResidentH1F32 = 2 * kTdtHidden, kTdtR
                    kTdtResidentWords = kTdtResidentHead + 2 * kTdtResidentBest;
 struct TdtResident {
   uint32_t* sync;        // per launch: arrival count, abort flag, each kTdtSyncStride words apart
-  uint64_t* exchange;    // [batch, kTdtResidentWords], right after the sync words; cleared per decode
+  uint64_t* exchange;    // [batch, kTdtResidentWords], behind the sync words of the launches and of `team`
+                         // (its counters and flags for the op's batch); all cleared per decode
+  TdtTeam team;          // decodes the windows of abandoned launches (members 0: one workgroup each does)
   uint32_t base, windows;  // of one launch
   uint32_t spin_limit;   // polls before a wait gives up
   uint64_t join_ticks;   // 100 MHz ticks before the members stop waiting for each other at the start (0: at once)

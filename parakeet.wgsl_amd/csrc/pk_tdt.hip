@@ -226,7 +226,7 @@ template <class P>
 __global__ __launch_bounds__(kTdtThreads) void tdt_decode_kernel(TdtArgs a) {
   __shared__ Shared<P> s;
   const uint32_t b = blockIdx.x, t = threadIdx.x;
-  if (a.aborted && a.aborted[2 * (b / a.aborted_windows) * kTdtSyncStride] == 0u) return;
+  if (decoded_before(a, b)) return;
   float* state = a.state + (uint64_t)b * 4 * H;
   float* cand = a.scratch + (uint64_t)b * 5 * H;
   const typename P::W* encoder = wptr<P>(a.encoder) + (uint64_t)b * a.frames * H;
@@ -744,6 +744,7 @@ __global__ __launch_bounds__(kTdtTeamThreads) void tdt_team_kernel(TdtArgs a, Td
   __shared__ TeamShared s;
   const uint32_t P = tm.members;
   const uint32_t b = blockIdx.x / P, p = blockIdx.x % P, t = threadIdx.x;
+  if (decoded_before(a, b)) return;
   const uint32_t U = H / P, u0 = p * U;
   const uint32_t hq0 = p * (kTdtHead / 4) / P, hq1 = (p + 1) * (kTdtHead / 4) / P;
   float* state = a.state + (uint64_t)b * 4 * H;
@@ -880,16 +881,18 @@ uint32_t tdt_team_capacity(int device) {
 }
 
 hipError_t launch_tdt_team(const TdtArgs& args, const TdtTeam& team, uint32_t batch, hipStream_t stream,
-                           hipEvent_t start, hipEvent_t stop) {
+                           hipEvent_t start, hipEvent_t stop, bool cleared) {
   if (batch == 0) return hipSuccess;
   if (!tdt_team_members_supported(team.members) || batch > team.capacity) return hipErrorInvalidValue;
   int device = 0;
   hipError_t e = hipGetDevice(&device);
   if (e != hipSuccess) return e;
   if ((uint64_t)batch * team.members > tdt_team_capacity(device)) return hipErrorInvalidConfiguration;
-  const uint32_t words = 2 * team.capacity * kTdtSyncStride;
-  hipLaunchKernelGGL(tdt_team_clear, dim3((words + 255) / 256), dim3(256), 0, stream, team.sync, words);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
+  if (!cleared) {
+    const uint32_t words = 2 * team.capacity * kTdtSyncStride;
+    hipLaunchKernelGGL(tdt_team_clear, dim3((words + 255) / 256), dim3(256), 0, stream, team.sync, words);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
   const dim3 grid(batch * team.members), block(kTdtTeamThreads);
   if (start || stop)
     hipExtLaunchKernelGGL(tdt_team_kernel, grid, block, 0, stream, start, stop, 0, args, team);

@@ -18,9 +18,11 @@ struct pk_tdt_op {
   uint32_t batch = 0;
   pk::TdtArgs args{};
   bool f32 = false;     // the f32 profile (no teams)
-  pk::TdtTeam team{};   // members == 0: one workgroup per window
-  uint32_t* team_memory = nullptr;
-  pk::TdtResident resident{};  // sync null: the team's or the window's own workgroups decode
+  // The memory behind one of: a team decode, a resident decode with (f16) the
+  // team that takes its abandoned launches, neither (one workgroup per window).
+  uint32_t* memory = nullptr;
+  pk::TdtTeam team{};          // members == 0: no team decode
+  pk::TdtResident resident{};  // sync null: no resident decode
   bool resident_decoded = false;  // a resident decode was enqueued: its abort words mean something
   bool destroyed = false;
 };
@@ -103,56 +105,79 @@ uint32_t choose_members(int device, uint32_t batch, bool f32) {
   return 0;
 }
 
-// Frees the team buffers once no launch can still use them (hipFree alone
+// Frees the op's buffers once no launch can still use them (hipFree alone
 // would not order the free after work enqueued on another stream).
-void free_team(pk_tdt_op* op) {
-  if (op->team_memory || op->resident.sync) {
+void free_buffers(pk_tdt_op* op) {
+  if (op->memory) {
     (void)hipSetDevice(op->ctx->device);
     (void)hipDeviceSynchronize();
-    (void)hipFree(op->team_memory);
-    (void)hipFree(op->resident.sync);
+    (void)hipFree(op->memory);
   }
-  op->team_memory = nullptr;
+  op->memory = nullptr;
   op->team = pk::TdtTeam{};
   op->resident = pk::TdtResident{};
   op->resident_decoded = false;
 }
 
-// Gives an op whose team size was left to the library (0) the resident
-// decode, where the device holds its workgroups and the batch takes at most
-// kTdtResidentLaunches launches. Without memory for its exchange words (34
-// KB per window) the op decodes with the chosen team, as it does elsewhere.
-int set_resident(pk_tdt_op* op) {
-  const uint64_t windows = (uint64_t)pk::kTdtResidentLaunches * pk::tdt_resident_windows(op->f32);
-  if (op->batch > windows || op->ctx->device < 0 || op->ctx->device >= kMaxDevices || !pk::tdt_resident_fits(op->ctx->device, op->f32)) return PK_OK;
-  const uint64_t sync_words = 2ull * pk::kTdtResidentLaunches * pk::kTdtSyncStride;
-  uint32_t* memory = nullptr;
-  if (hipMalloc(reinterpret_cast<void**>(&memory), sync_words * 4 + (uint64_t)op->batch * pk::kTdtResidentWords * 8) !=
-      hipSuccess) {
-    (void)hipGetLastError();
-    return PK_OK;
-  }
-  op->resident.sync = memory;
-  op->resident.exchange = reinterpret_cast<uint64_t*>(memory + sync_words);
-  op->resident.spin_limit = 1u << 20;    // each a memory round trip: about a second
-  op->resident.join_ticks = 1000000;     // 10 ms
-  return PK_OK;
+uint64_t team_sync_words(const pk_tdt_op* op, uint32_t members) {
+  return members ? 2ull * op->batch * pk::kTdtSyncStride : 0;
+}
+uint64_t team_partial_words(const pk_tdt_op* op, uint32_t members) { return (uint64_t)op->batch * 2 * members * 4; }
+
+pk::TdtTeam team_of(const pk_tdt_op* op, uint32_t members, uint32_t* sync, uint32_t* partials, uint32_t spin_limit) {
+  pk::TdtTeam t{};
+  t.members = members;
+  t.sync = sync;
+  t.partials = partials;
+  t.capacity = op->batch;
+  t.spin_limit = spin_limit;
+  return t;
 }
 
 int set_team(pk_tdt_op* op, uint32_t members) {
-  free_team(op);
+  free_buffers(op);
   if (members == 0) return PK_OK;
-  const uint64_t sync_words = 2ull * op->batch * pk::kTdtSyncStride;
-  const uint64_t words = sync_words + (uint64_t)op->batch * 2 * members * 4;
-  const hipError_t e = hipMalloc(reinterpret_cast<void**>(&op->team_memory), words * 4);
+  const uint64_t sync_words = team_sync_words(op, members);
+  const hipError_t e =
+      hipMalloc(reinterpret_cast<void**>(&op->memory), (sync_words + team_partial_words(op, members)) * 4);
   if (e != hipSuccess)
     return fail(PK_ALLOCATION_FAILURE, "%s: cannot allocate the decoder's team buffers: %s", op->label.c_str(),
                 hipGetErrorString(e));
-  op->team.members = members;
-  op->team.sync = op->team_memory;
-  op->team.partials = op->team_memory + sync_words;
-  op->team.capacity = op->batch;
-  op->team.spin_limit = 1u << 24;
+  op->team = team_of(op, members, op->memory, op->memory + sync_words, 1u << 24);
+  return PK_OK;
+}
+
+// The decode of an op whose team size is left to the library: the resident
+// one where the device holds its workgroups and the batch takes at most
+// kTdtResidentLaunches launches, else (also without memory for its exchange
+// words, 34 KB per window) the team size that choose_members finds.
+int set_chosen(pk_tdt_op* op) {
+  const int device = op->ctx->device;
+  const uint32_t members = choose_members(device, op->batch, op->f32);
+  const uint64_t windows = (uint64_t)pk::kTdtResidentLaunches * pk::tdt_resident_windows(op->f32);
+  if (op->batch > windows || device < 0 || device >= kMaxDevices || !pk::tdt_resident_fits(device, op->f32))
+    return set_team(op, members);
+  free_buffers(op);
+  const uint64_t sync_words = 2ull * pk::kTdtResidentLaunches * pk::kTdtSyncStride;
+  const uint64_t exchange_at = sync_words + team_sync_words(op, members);
+  const uint64_t partials_at = exchange_at + (uint64_t)op->batch * pk::kTdtResidentWords * 2;
+  if (hipMalloc(reinterpret_cast<void**>(&op->memory), (partials_at + team_partial_words(op, members)) * 4) !=
+      hipSuccess) {
+    (void)hipGetLastError();
+    op->memory = nullptr;
+    return set_team(op, members);
+  }
+  op->resident.sync = op->memory;
+  op->resident.exchange = reinterpret_cast<uint64_t*>(op->memory + exchange_at);
+  op->resident.spin_limit = 1u << 20;  // each a memory round trip: about a second
+  // Waiting for other work to leave its compute units pays up to about what the
+  // kernels behind an abandoned launch take, 3-18 ms (f16), 5-46 ms (f32).
+  // Beside a decode of 100 windows with one workgroup each (19 ms, its
+  // workgroups end one by one) one f16 window takes 5.8 ms, 11.3 with 2 ms of
+  // patience; 16 windows 9.6 and 25.5.
+  op->resident.join_ticks = op->f32 ? 2000000 : 1000000;  // 20 and 10 ms
+  // The teams do not insist either (some 0.1 s): behind them is a kernel that never waits.
+  op->resident.team = team_of(op, members, op->memory + sync_words, op->memory + partials_at, 1u << 16);
   return PK_OK;
 }
 
@@ -269,10 +294,7 @@ int pk_tdt_create(pk_context* ctx, const pk_tdt_desc* d, pk_tdt_op** out) {
   op->batch = d->batch_size;
   op->args = args_of(d);
   op->f32 = d->precision == PK_PRECISION_F32;
-  int st = set_team(op, choose_members(ctx->device, op->batch, op->f32));
-  if (st == PK_OK) st = set_resident(op);
-  if (st != PK_OK) {
-    free_team(op);
+  if (int st = set_chosen(op)) {
     delete op;
     return st;
   }
@@ -284,9 +306,11 @@ int pk_tdt_set_team_size(pk_tdt_op* op, uint32_t members) {
   if (!op) return fail(PK_INVALID_ARGUMENT, "TDT decoder op is null");
   if (op->destroyed) return fail(PK_DESTROYED, "%s was destroyed", op->label.c_str());
   PK_HIP(hipSetDevice(op->ctx->device), "hipSetDevice");
-  const bool chosen = members == 0;
-  if (chosen) members = choose_members(op->ctx->device, op->batch, op->f32);
-  else if (members == 1) members = 0;
+  if (members == 0) {
+    if (int s = set_chosen(op)) return s;
+    return ok();
+  }
+  if (members == 1) members = 0;
   else if (!pk::tdt_team_members_supported(members))
     return fail(PK_RANGE_ERROR, "%s team size must be 0, 1, 8 or 16", op->label.c_str());
   else if (op->f32)
@@ -296,12 +320,13 @@ int pk_tdt_set_team_size(pk_tdt_op* op, uint32_t members) {
     return fail(PK_RANGE_ERROR, "%s: %u windows x %u workgroups cannot be resident together", op->label.c_str(),
                 op->batch, members);
   if (int s = set_team(op, members)) return s;
-  return chosen ? set_resident(op) : PK_OK;
+  return ok();
 }
 
 int pk_tdt_team_size(const pk_tdt_op* op, uint32_t* members) {
   if (!op || !members) return fail(PK_INVALID_ARGUMENT, "TDT decoder op or output is null");
-  *members = op->team.members ? op->team.members : 1u;
+  const uint32_t own = op->resident.sync ? op->resident.team.members : op->team.members;
+  *members = own ? own : 1u;
   return ok();
 }
 
@@ -322,6 +347,13 @@ int pk_tdt_set_join_limit(pk_tdt_op* op, uint32_t ticks) {
   if (!op) return fail(PK_INVALID_ARGUMENT, "TDT decoder op is null");
   if (op->destroyed) return fail(PK_DESTROYED, "%s was destroyed", op->label.c_str());
   op->resident.join_ticks = ticks;
+  return ok();
+}
+
+int pk_tdt_set_team_limit(pk_tdt_op* op, uint32_t polls) {
+  if (!op) return fail(PK_INVALID_ARGUMENT, "TDT decoder op is null");
+  if (op->destroyed) return fail(PK_DESTROYED, "%s was destroyed", op->label.c_str());
+  op->resident.team.spin_limit = polls;
   return ok();
 }
 
@@ -381,7 +413,7 @@ int pk_tdt_enqueue_timed(pk_tdt_op* op, uint32_t active_batch, void* stream, voi
 int pk_tdt_destroy(pk_tdt_op* op) {
   if (!op || op->destroyed) return ok();
   op->destroyed = true;
-  free_team(op);
+  free_buffers(op);
   return ok();
 }
 

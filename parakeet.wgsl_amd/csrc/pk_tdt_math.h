@@ -85,6 +85,12 @@ __device__ __forceinline__ A4 bias4(const float* p) {
   return A4{(E)b.x, (E)b.y, (E)b.z, (E)b.w};
 }
 
+// Whether a kernel behind resident launches leaves window b as it is.
+__device__ __forceinline__ bool decoded_before(const TdtArgs& a, uint32_t b) {
+  return a.aborted && (a.aborted[2 * (b / a.aborted_windows) * kTdtSyncStride] == 0u ||
+                       (a.after_team && !(a.status[b] & kTdtSyncTimeout)));
+}
+
 // Exchanged values: relaxed agent-scope atomics, coherent between XCDs.
 __device__ __forceinline__ float xload(const float* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

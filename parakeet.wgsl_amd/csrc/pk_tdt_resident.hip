@@ -32,10 +32,12 @@
 // Residency. Members poll, so all of them must be resident. Each counts
 // itself in and waits until the count is full or a bounded time has passed;
 // then it raises the abort flag and everyone leaves, as it does when a later
-// poll exceeds its limit. The kernel that follows in the stream
-// (tdt_decode_kernel, one workgroup per window, no waiting) decodes every
-// window of an aborted launch from the start and does nothing otherwise, so a
-// device busy with other work costs time, never a result.
+// poll exceeds its limit. The kernels that follow in the stream decode every
+// window of an aborted launch from the start and do nothing otherwise: in f16
+// tdt_team_kernel, whose small workgroups fit beside others where these do
+// not, and for windows whose team gives up too (every f32 one)
+// tdt_decode_kernel, one workgroup per window without any waiting. So a device
+// busy with other work costs time, never a result.
 //
 // Measured on whole decodes of 188 frames, synthetic weights, against the
 // kernels of pk_tdt.hip that ran before (the longest window has 63 tokens for
@@ -1074,7 +1076,8 @@ hipError_t launch_tdt_resident(const TdtArgs& args, const TdtResident& resident,
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)plan.lds_bytes);
   if (e != hipSuccess) return e;
   // the sync words precede the exchanged ones: one range to clear
-  const uint32_t units = (2 * kTdtResidentLaunches * kTdtSyncStride * 4 + batch * kTdtResidentWords * 8) / 16;
+  const uint32_t units =
+      (uint32_t)(resident.exchange + (uint64_t)batch * kTdtResidentWords - reinterpret_cast<uint64_t*>(resident.sync)) / 2;
   hipLaunchKernelGGL(tdt_resident_clear, dim3(min((units + 255) / 256, 1024u)), dim3(256), 0, stream,
                      reinterpret_cast<uint4*>(resident.sync), units);
   if ((e = hipGetLastError()) != hipSuccess) return e;
@@ -1090,10 +1093,14 @@ hipError_t launch_tdt_resident(const TdtArgs& args, const TdtResident& resident,
       hipLaunchKernelGGL(plan.kernel, dim3(plan.members), dim3(kBlock), plan.lds_bytes, stream, args, r);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  // windows of an aborted launch, one workgroup each; none otherwise
+  // windows of an aborted launch; none otherwise
   TdtArgs again = args;
   again.aborted = resident.sync + kTdtSyncStride;
   again.aborted_windows = per_launch;
+  if (resident.team.members) {
+    if ((e = launch_tdt_team(again, resident.team, batch, stream, nullptr, nullptr, true)) != hipSuccess) return e;
+    again.after_team = 1;
+  }
   return launch_tdt_decode(again, batch, f32, stream, nullptr, stop);
 }
 

@@ -552,6 +552,7 @@ SIGNATURES = {
     "pk_tdt_abandoned_launches": (ctypes.c_int, [_VP, ctypes.POINTER(ctypes.c_uint32)]),
     "pk_tdt_set_wait_limit": (ctypes.c_int, [_VP, ctypes.c_uint32]),
     "pk_tdt_set_join_limit": (ctypes.c_int, [_VP, ctypes.c_uint32]),
+    "pk_tdt_set_team_limit": (ctypes.c_int, [_VP, ctypes.c_uint32]),
     "pk_graph_begin_capture": (ctypes.c_int, [_VP, _VP]),
     "pk_graph_end_capture": (ctypes.c_int, [_VP, _VP, _PPV]),
     "pk_graph_launch": (ctypes.c_int, [_VP, _VP]),
@@ -1280,12 +1281,16 @@ class TdtDecoderOp:
         return out.value
 
     def set_wait_limit(self, polls: int) -> None:
-        """Polls before a resident launch is given up (and decoded by one workgroup per window)."""
+        """Polls before a resident launch is given up (and decoded by the kernels behind it)."""
         check(load().pk_tdt_set_wait_limit(self.handle, polls))
 
     def set_join_limit(self, ticks: int) -> None:
         """100 MHz ticks a resident launch waits for its workgroups at the start (0: given up)."""
         check(load().pk_tdt_set_join_limit(self.handle, ticks))
+
+    def set_team_limit(self, polls: int) -> None:
+        """Polls of a barrier of the teams behind a resident launch before they give up too."""
+        check(load().pk_tdt_set_team_limit(self.handle, polls))
 
     def destroy(self) -> None:
         check(load().pk_tdt_destroy(self.handle))

@@ -1,8 +1,8 @@
 """The resident TDT decode (weights in LDS, every window of a launch sharing
 them) against the decode with one workgroup per window: bit-identical
 tokens, states and scratch at the edges of its launch shapes, with head
-weights that are not finite, on two streams at once, and when its workgroups
-give up waiting."""
+weights that are not finite, on two streams at once, and when its workgroups,
+or those and the teams behind them, give up waiting."""
 import numpy as np
 import pytest
 
@@ -39,7 +39,7 @@ class Decoder:
         return {n: b.download().view(np.uint32) for n, b in self.out.items()}
 
 
-def decode(abi, scope, ctx, case, precision, *, team=None, polls=None, join=None, active=0):
+def decode(abi, scope, ctx, case, precision, *, team=None, polls=None, join=None, team_polls=None, active=0):
     d = Decoder(abi, scope, ctx, case, precision)
     try:
         if team is not None:
@@ -49,6 +49,8 @@ def decode(abi, scope, ctx, case, precision, *, team=None, polls=None, join=None
             d.op.set_wait_limit(polls)
         if join is not None:
             d.op.set_join_limit(join)
+        if team_polls is not None:
+            d.op.set_team_limit(team_polls)
         print(precision, "batch", case.batch, "team", team, "polls", polls, "join", join, flush=True)
         assert d.op.abandoned_launches() == 0
         d.op.enqueue(active)
@@ -96,11 +98,14 @@ def test_resident_decode_leaves_out_zero_inputs_of_weights_that_are_not_finite(a
     same(decode(abi, scope, ctx, case, precision), decode(abi, scope, ctx, case, precision, team=1))
 
 
+@pytest.mark.parametrize("team_polls", [None, 0])  # the teams behind it decode, or give up as well
 @pytest.mark.parametrize("limit", ["polls", "join"])
 @pytest.mark.parametrize("precision,batch", [("f16", 3), ("f16", 33), ("f32", 7)])
-def test_resident_decode_that_gives_up_is_decoded_again(abi, ctx, scope, workloads, precision, batch, limit):
+def test_resident_decode_that_gives_up_is_decoded_again(abi, ctx, scope, workloads, precision, batch, limit,
+                                                                team_polls):
     case = ragged(workloads, 40 + batch, batch, precision, 0.5)
-    same(decode(abi, scope, ctx, case, precision, **{limit: 0}), decode(abi, scope, ctx, case, precision, team=1))
+    same(decode(abi, scope, ctx, case, precision, team_polls=team_polls, **{limit: 0}),
+         decode(abi, scope, ctx, case, precision, team=1))
 
 
 def test_resident_decodes_on_two_streams_and_an_active_prefix(abi, ctx, scope, workloads):
