@@ -479,16 +479,9 @@ struct Wave {
   __device__ __forceinline__ void cell(int layer, Acc acc, bool need) {
     float ig, fg, gg, og;
     const int base = (int)(lane - part);
+    static_assert(kPacked == (C == 2), "an f16 lane has two gates, an f32 lane one");
     if constexpr (C == 1) {
-      float sum;
-      if constexpr (kPacked) {
-        const uint32_t bits = __builtin_bit_cast(uint16_t, acc);
-        const _Float16 other =
-            __builtin_bit_cast(_Float16, (uint16_t)(uint32_t)__shfl_xor((int)bits, 1, 64));
-        sum = (float)(_Float16)(acc + other);
-      } else {
-        sum = acc + __shfl_xor(acc, 1, 64);
-      }
+      const float sum = acc + __shfl_xor(acc, 1, 64);
       const float act = activate(sum, (part >> 1) == 2u);
       ig = __shfl(act, base, 64);
       fg = __shfl(act, base + 2, 64);
