@@ -1533,13 +1533,22 @@ static napi_value js_tdt_set_team_size(napi_env env, napi_callback_info info) {
   return undefined(env);
 }
 
-/* tdtTeamSize(op) -> workgroups per window of the next launch */
+/* tdtTeamSize(op) -> workgroups per window of the team decode (1: no team) */
 static napi_value js_tdt_team_size(napi_env env, napi_callback_info info) {
   napi_value argv[1];
   uint32_t members = 0;
   if (!get_args(env, info, 1, argv)) return NULL;
   PK_CALL(env, pk_tdt_team_size((const pk_tdt_op *)get_external(env, argv[0]), &members));
   return make_number(env, members);
+}
+
+/* tdtResidentWindows(op) -> windows of one resident launch (0: not that decode) */
+static napi_value js_tdt_resident_windows(napi_env env, napi_callback_info info) {
+  napi_value argv[1];
+  uint32_t windows = 0;
+  if (!get_args(env, info, 1, argv)) return NULL;
+  PK_CALL(env, pk_tdt_resident_windows((const pk_tdt_op *)get_external(env, argv[0]), &windows));
+  return make_number(env, windows);
 }
 
 static napi_value js_tdt_destroy(napi_env env, napi_callback_info info) {
@@ -1612,6 +1621,7 @@ static napi_value init(napi_env env, napi_value exports) {
       {"tdtDestroy", js_tdt_destroy},
       {"tdtSetTeamSize", js_tdt_set_team_size},
       {"tdtTeamSize", js_tdt_team_size},
+      {"tdtResidentWindows", js_tdt_resident_windows},
   };
   for (size_t i = 0; i < sizeof fns / sizeof fns[0]; ++i) {
     napi_value f;

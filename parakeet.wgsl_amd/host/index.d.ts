@@ -597,9 +597,11 @@ export interface TdtDecoderDescriptor {
 /** tdt-decoder.ts:84-137 */
 export declare class TdtDecoderDispatch {
   readonly label: string;
-  /** Workgroups per window of the next launch (this library only). */
+  /** Windows of one resident launch, 0 if it does not decode that way (this library only). */
+  readonly residentWindows: number;
+  /** Workgroups per window of the team decode, 1 without a team: what runs where residentWindows is 0 (this library only). */
   readonly teamSize: number;
-  /** 0 chooses, 1 one workgroup per window, 8 or 16 a team (this library only). */
+  /** 0 leaves it to the library (resident where it applies), 1 one workgroup per window, 8 or 16 a team (this library only). */
   setTeamSize(members: number): void;
   encode(encoder: HipCommandEncoder, timestampWrites?: TimestampWrites, activeBatchSize?: number): void;
   destroy(): void;

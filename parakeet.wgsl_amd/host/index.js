@@ -1838,12 +1838,28 @@ class TdtDecoderDispatch {
     native().tdtDestroy(this.op);
   }
 
-  /** Workgroups per window of the next launch (no reference counterpart). */
+  /**
+   * Windows that one launch of the resident decode takes, its weights in the
+   * LDS of most compute units; 0 if the dispatch does not decode that way (no
+   * reference counterpart).
+   */
+  get residentWindows() {
+    return native().tdtResidentWindows(this.op);
+  }
+
+  /**
+   * Workgroups per window of the team decode, 1 without a team: what the next
+   * launch runs where residentWindows is 0, and what takes the windows of a
+   * resident launch that gives up (no reference counterpart).
+   */
   get teamSize() {
     return native().tdtTeamSize(this.op);
   }
 
-  /** 0 chooses, 1 one workgroup per window, 8 or 16 a team (no reference counterpart). */
+  /**
+   * 0 leaves the decode to the library (resident where it applies), 1 runs one
+   * workgroup per window, 8 or 16 a team (no reference counterpart).
+   */
   setTeamSize(members) {
     native().tdtSetTeamSize(this.op, members);
   }
@@ -1853,8 +1869,7 @@ class TdtDecoderDispatch {
  * PersistentTdtDecoderKernel (tdt-decoder.ts:139-366): greedy TDT decoding
  * with the whole autoregressive loop inside one launch, over the package's
  * resident decoder shard; the fp16 profile (f16 weights and encoder rows)
- * or the fp32 profile (f32 weights and encoder rows, one workgroup per
- * window).
+ * or the fp32 profile (f32 weights and encoder rows, no teams).
  */
 class PersistentTdtDecoderKernel {
   constructor(device, arena, weights, precision) {

@@ -72,6 +72,12 @@ async function main() {
   const expectedTeam = precision === "fp32" ? 1 : 16;
   if (dispatch.teamSize !== expectedTeam)
     throw new Error(`decoder ran with team size ${dispatch.teamSize}, expected ${expectedTeam}`);
+  const expectedResident = precision === "fp32" ? 6 : 16;
+  if (dispatch.residentWindows !== expectedResident)
+    throw new Error(`resident launches of ${dispatch.residentWindows} windows, expected ${expectedResident}`);
+  dispatch.setTeamSize(1);
+  if (dispatch.residentWindows !== 0 || dispatch.teamSize !== 1)
+    throw new Error("team size 1 still decodes another way");
   dispatch.destroy();
   dispatch.destroy();
   arena.destroy();
