@@ -185,3 +185,10 @@ def test_roofline_slots_pick_both_ff_modules():
     with pytest.raises(SystemExit, match="dispatch slots"):
         bench.roofline_slots(layers, 1, "projector", dispatches, launches + 1)
 
+
+
+def test_peak_of_the_units_a_kernel_runs_on():
+    """An f32 GEMM is six bf16 products, f32 attention runs on the f32 units."""
+    assert bench.peak_tflops("f32", "feed-forward1-linear1") == pytest.approx(2500 / 6)
+    assert bench.peak_tflops("f32", "relative-attention") == 157.3
+    assert bench.peak_tflops("f16", "relative-attention") == bench.peak_tflops("f16", "projector") == 2500.0
