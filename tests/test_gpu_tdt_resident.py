@@ -6,6 +6,7 @@ or those and the teams behind them, give up waiting."""
 import numpy as np
 import pytest
 
+from test_gpu_encoder import Stack
 from test_gpu_parity import Scope
 
 pytestmark = pytest.mark.gpu
@@ -131,3 +132,30 @@ def test_resident_decodes_on_two_streams_and_an_active_prefix(abi, ctx, scope, w
             d.op.release()
         abi.check(abi.load().pk_stream_destroy(ctx.handle, other))
     same(decode(abi, scope, ctx, cases[0], "f16", active=5), decode(abi, scope, ctx, cases[0], "f16", team=1, active=5))
+
+
+@pytest.mark.parametrize("precision", ["f16", "f32"])
+def test_resident_decode_beside_encoder_passes(abi, ctx, scope, workloads, precision):
+    """Decodes on one stream while encoder passes run on another: both as when
+    alone, to the bit, and no launch is given up for the passes' sake."""
+    case = ragged(workloads, 80, 6, precision, 0.5)
+    want = decode(abi, scope, ctx, case, precision, team=1)
+    encoder = Stack(abi, ctx, scope, workloads.encoder_stack(seed=81, windows=8, frames=188, layers=2))
+    decoder = Decoder(abi, scope, ctx, case, precision)
+    other = abi.ctypes.c_void_p()
+    abi.check(abi.load().pk_stream_create(ctx.handle, abi.ctypes.byref(other)))
+    try:
+        alone = encoder.run(graph=True)
+        for _ in range(4):
+            encoder.op.enqueue(graph=True)
+            decoder.op.enqueue(0, other)
+            encoder.op.enqueue(graph=True)
+        ctx.synchronize()
+        ctx.synchronize(other)
+        assert decoder.op.abandoned_launches() == 0
+        same(decoder.words(), want)
+        np.testing.assert_array_equal(encoder.output.download().view(np.uint16), alone.view(np.uint16))
+    finally:
+        decoder.op.release()
+        encoder.release()
+        abi.check(abi.load().pk_stream_destroy(ctx.handle, other))
