@@ -337,9 +337,10 @@ __global__ __launch_bounds__(64 * WN * KS, 2) void gemm_f32_kernel(GemmArgs args
         read_a(buf, 1, a1);
         multiply(w, a0);
         // ahead of the split, whose chain a wave alone on its SIMD waits for
-        // (96 x 128, 512 x 4096 -> 1024: 122.7 us, 127.0 inside it)
+        // (96 x 128, 512 x 4096 -> 1024: 122.7 us, 127.0 inside it), but not
+        // with one row block (6-bit 256 x 1024 -> 1024 21.3 us, 20.3 inside)
         const uint32_t next = min(t + 2u, steps - 1u);
-        scale_a(next, a_stage[half]);
+        if constexpr (MB > 1) scale_a(next, a_stage[half]);
         assemble(e, w);
         if (half == 0)
           gather(cw, 2, sign, e);
@@ -348,6 +349,7 @@ __global__ __launch_bounds__(64 * WN * KS, 2) void gemm_f32_kernel(GemmArgs args
         // three row blocks: the split of the new rows first (3008 x 4096 -> 1024
         // 143 us against 146; 32 x 128 and 64 x 256 lose 2% and 10% that way)
         if constexpr (MB < 3) read_a(buf1, 0, a0);
+        if constexpr (MB == 1) scale_a(next, a_stage[half]);
         store_a(buf2, a_stage[half]);
         load_a(min(t + 4u, steps - 1u), a_stage[half]);
         if constexpr (MB >= 3) read_a(buf1, 0, a0);
