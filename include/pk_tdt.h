@@ -160,8 +160,10 @@ int pk_tdt_release(pk_tdt_op *op);
    that allocates nothing, for callers that cannot allocate device memory
    (code under HIP graph capture, tight serving loops, harnesses that forbid
    hipMalloc). It validates like pk_tdt_create, then launches like
-   pk_tdt_enqueue of every window with team size `members` (0 chooses, 1,
-   8 or 16; bit-identical results for each), taking the team's barrier
+   pk_tdt_enqueue of every window with team size `members` (0: the size that
+   pk_tdt_team_size reports for so many windows; 1, 8 or 16; bit-identical
+   results for each, never the resident decode, which needs memory of an op),
+   taking the team's barrier
    counters and argmax partials from a static device array of the library
    (64 KB per GPU, held until the process ends) instead of buffers of an
    op. At most PK_TDT_STATIC_MAX_WINDOWS windows (PK_RANGE_ERROR beyond).
