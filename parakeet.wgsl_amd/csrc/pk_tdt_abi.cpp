@@ -198,9 +198,10 @@ hipError_t launch_in_turn(const pk_tdt_op* op, uint32_t batch, hipStream_t strea
     e = hipStreamWaitEvent(stream, turn.last, 0);
   else
     e = hipEventCreateWithFlags(&turn.last, hipEventDisableTiming);
-  if (e == hipSuccess) e = pk::launch_tdt_resident(op->args, op->resident, batch, op->f32, stream, start, stop);
-  if (e == hipSuccess) e = hipEventRecord(turn.last, stream);
-  return e;
+  if (e != hipSuccess) return e;
+  e = pk::launch_tdt_resident(op->args, op->resident, batch, op->f32, stream, start, stop);
+  const hipError_t recorded = hipEventRecord(turn.last, stream);  // a refused launch may have others before it
+  return e == hipSuccess ? recorded : e;
 }
 
 // Kernel arguments of a validated descriptor.
