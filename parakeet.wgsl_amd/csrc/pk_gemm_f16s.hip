@@ -13,11 +13,11 @@
 // wavefront, as one coalesced 16-byte + one 4/8-byte load per lane and
 // column block of the operand-order stream (the package's own bits per
 // code, no larger layout). Activation fragments come straight from global
-// memory (a few hundred KB, L2-resident; past 32 rows the 32 x 32 tile turns
-// whole rows into fragments through LDS instead); a wavefront reuses each fragment
-// for its CB column blocks, so the activation bytes a workgroup pulls from
-// L2 are 3.2 * RW / CB times its weight bytes (5-bit). The K loop has no
-// LDS tile and no barrier: a wavefront issues the loads of its next K
+// memory (a few hundred KB, L2-resident; past 32 rows and from K = 768 on the
+// 32 x 32 tile turns whole rows into fragments through LDS instead); a
+// wavefront reuses each fragment for its CB column blocks, so the activation
+// bytes a workgroup pulls from L2 are 3.2 * RW / CB times its weight bytes
+// (5-bit). The K loop has no shared LDS tile and no barrier: a wavefront issues the loads of its next K
 // block, decodes the current one (shift/mask/v_alignbit per code, palette
 // gather from LDS) into MFMA operands and runs the MFMAs. The W partial
 // tiles are summed through LDS in wavefront order (deterministic), then

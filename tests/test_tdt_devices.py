@@ -68,7 +68,8 @@ def test_queries_go_to_the_ops_own_device(abi, tmp_path):
     source, stub = tmp_path / "hip_stub.c", tmp_path / "hip_stub.so"
     source.write_text(STUB)
     subprocess.run(["gcc", "-shared", "-fPIC", "-w", str(source), "-o", str(stub)], check=True)
-    env = dict(os.environ, LD_PRELOAD=str(stub), PYTHONPATH=ROOT)
+    preload = ":".join(p for p in (str(stub), os.environ.get("LD_PRELOAD")) if p)
+    env = dict(os.environ, LD_PRELOAD=preload, PYTHONPATH=ROOT)
     child = subprocess.run([sys.executable, "-c", CHILD, str(stub)], cwd=ROOT, env=env, capture_output=True, text=True,
                            timeout=120)
     assert child.returncode == 0, child.stdout + child.stderr
